@@ -9,6 +9,7 @@
 
 #include <algorithm>
 #include <array>
+#include <cmath>
 #include <cstdarg>
 #include <initializer_list>
 #include <cstdio>
@@ -89,6 +90,7 @@ enum ScratchSlot {
   SC_PLN,   // sublayer (host call): post_ln staged
   SC_XL,    // latent MoE: x projected down
   SC_ROUTED,  // latent MoE: summed routed rows
+  SC_XP,      // batches: partial sums of the K parts
   SC_MIXA,    // mixers: the GDN conv output / the GQA prepared queries
   SC_MIXB,    // mixers: the GQA softmax partials
   SC_N
@@ -114,12 +116,14 @@ struct Layer {
   size_t shared_gs = 0, shared_inter = 0;
   int routed_kind = -1;
   size_t routed_gs = 0;
+  bool al16 = false;  // every routed (and the shared) expert's pointers are 16-byte aligned
   // the latent MoE's view of the pool at (moe_hidden, moe_inter): n_experts jobs, then a zero job
   bool lat_dirty = true;
   RbtExpertDev *d_lat = nullptr;
   size_t lat_cap = 0, lat_mh = 0;
   int lat_kind = -1;
   size_t lat_gs = 0;
+  bool lat_al16 = false;
 };
 
 }  // namespace
@@ -258,6 +262,42 @@ int scratch_t(rbt_ctx *c, int slot, size_t count, T **out) {
   return RBT_OK;
 }
 
+// Whether the call can have these scratch sizes: they fit the fixed array of an allocation-free call,
+// or the slots are large enough or can grow now (a stream under capture allocates nothing). False
+// leaves the call as it was, for a path that needs less.
+bool scratch_avail(rbt_ctx *c, std::initializer_list<std::pair<int, size_t>> need) {
+  if (c->arena) {
+    size_t sum = 0;
+    for (const auto &n : need) {
+      if (c->arena_sz[n.first] == 0) sum += align256(std::max<size_t>(n.second, 1));
+      else if (c->arena_sz[n.first] < n.second) return false;
+    }
+    return sum <= c->arena_cap - c->arena_used;
+  }
+  for (const auto &n : need) {
+    if (c->scratch[n.first] && c->scratch_cap[n.first] >= n.second) continue;
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(c->stream, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) {
+      (void)hipGetLastError();
+      return false;
+    }
+    void *p;
+    const std::string err = c->err;
+    if (scratch(c, n.first, n.second, &p) != RBT_OK) {
+      c->err = err;
+      return false;
+    }
+  }
+  return true;
+}
+
+bool al16(std::initializer_list<const void *> ps) {
+  uintptr_t m = 0;
+  for (const void *p : ps) m |= (uintptr_t)p;
+  return m % 16 == 0;
+}
+bool al16(const RbtExpertDev &e) { return al16({e.gd, e.gs, e.ud, e.us, e.dd, e.ds}); }
+
 // Bytes of a QT's data and scale arrays.
 size_t qt_data_bytes(const rbt_qt &w) {
   if (w.kind == RBT_QT_F32) return w.rows * w.cols * 4;
@@ -387,6 +427,45 @@ const PoolEntry *find_pool_slot(rbt_ctx *c, const rbt_expert_slot *s) {
   return nullptr;
 }
 
+// Whether a batch through one matrix takes the tiled matrix-core kernels (split, product, sum of the K
+// parts: about 14 us of launches) rather than the GEMV per token, whose time grows with s. us, GEMV
+// against tiled: int4 7168 x 3584 s = 2 19.3 / 16.7, 16 63.6 / 20.5, 512 1615 / 135; MXFP4 3584 x 3072
+// s = 4 9.7 / 14.3, 16 18.7 / 14.2, 64 55.5 / 21.2; 2048 x 8192 s = 4 10.0 / 14.0, 16 24.4 / 13.8.
+bool x3_matmul_wins(int kind, size_t s, size_t i, size_t o) {
+  return s >= 2 && s * i * o >= (size_t)(kind == RBT_QT_I4_GROUPED ? 50 : 100) * 1000000;
+}
+
+// Rows per tile: 32 where the rows of one matrix (or an expert, on average) go past 16.
+int x3_tch(size_t rows) { return rows > 16 ? 32 : 16; }
+
+// A batch through one matrix on the matrix cores (x3gemm.hip): the activations' exact parts, then the
+// products, K split where the row blocks alone would leave CUs idle. Returns 1 when the scratch it
+// needs cannot be had (the caller takes another path).
+int x3_matmul(rbt_ctx *c, float *y, const float *x, const rbt_qt *w, size_t s) {
+  const size_t i = w->cols, o = w->rows;
+  // the partial sums' bound over every s up to this one, so that a smaller batch never grows it
+  const size_t part = (64 * (size_t)c->num_cu / (o / 128) + s + 32) * o;
+  if (!scratch_avail(c, {{SC_XB, 6 * s * i}, {SC_XP, 4 * part}})) return 1;
+  __bf16 *xb3;
+  float *xp;
+  RBT_TRY(scratch_t(c, SC_XB, 3 * s * i, &xb3));
+  RBT_TRY(scratch_t(c, SC_XP, part, &xp));
+  rbt::X3Args A;
+  A.single.dd = (const uint8_t *)w->data;
+  A.single.ds = w->scale;
+  A.nrows = A.S = (int)s;
+  A.xb3 = xb3;
+  A.K = (int)i;
+  A.O = (int)o;
+  A.tch = x3_tch(s);
+  A.KS = rbt::x3_parts(*c, s, A.tch, i, o, false);
+  A.y = A.KS > 1 ? xp : y;
+  HIP_OK(c, rbt::launch_x3split(*c, w->kind, x, s, i, xb3));
+  HIP_OK(c, rbt::launch_x3(*c, w->kind, false, A));
+  if (A.KS > 1) HIP_OK(c, rbt::launch_x3sum(*c, xp, s * o, A.KS, y));
+  return RBT_OK;
+}
+
 // y[S,O] = x . W^T for one QT whose pointers are device memory.
 int matmul_dev(rbt_ctx *c, float *y, const float *x, const rbt_qt *w, size_t s) {
   RBT_TRY(check_qt(c, w, "matmul"));
@@ -399,6 +478,10 @@ int matmul_dev(rbt_ctx *c, float *y, const float *x, const rbt_qt *w, size_t s) 
     // one token on the matrix cores, the whole matrix in flight at once
     HIP_OK(c, rbt::launch_xgemv1(*c, (const uint8_t *)w->data, (const uint8_t *)w->scale, x, (int)i, (int)o, y));
     return RBT_OK;
+  }
+  if (x3_matmul_wins(w->kind, s, i, o) && 6 * s * i < ((size_t)1 << 32) && al16({x, y, w->data, w->scale}) && rbt::x3_ok(w->kind, w->group_size, i, o, false)) {
+    const int rc = x3_matmul(c, y, x, w, s);
+    if (rc <= 0) return rc;
   }
   if (w->kind != RBT_QT_F32 && aligned && rbt::decode_shape_ok(i, w->kind, w->group_size)) {
     RbtExpertDev one{};
@@ -476,6 +559,7 @@ int refresh_table(rbt_ctx *c, uint32_t layer, Layer &L) {
   RbtExpertDev *t = L.h_table.data();
   memset(t, 0, E * sizeof(RbtExpertDev));
   L.routed_kind = -1;
+  L.al16 = al16(L.h_shared);
   for (auto &kv : c->pool) {
     if ((uint32_t)(kv.first >> 32) != layer) continue;
     uint32_t eid = (uint32_t)kv.first;
@@ -483,6 +567,7 @@ int refresh_table(rbt_ctx *c, uint32_t layer, Layer &L) {
     int kind;
     size_t gs;
     RBT_TRY(slot_view(c, &kv.second.slot, L.desc.hidden, L.desc.moe_inter, &t[eid], &kind, &gs));
+    L.al16 = L.al16 && al16(t[eid]);
     if (L.routed_kind >= 0 && (kind != L.routed_kind || gs != L.routed_gs))
       return fail(c, RBT_E_UNSUPPORTED, "layer %u: routed experts mix weight formats", layer);
     L.routed_kind = kind;
@@ -503,6 +588,7 @@ int refresh_latent(rbt_ctx *c, uint32_t layer, Layer &L, size_t mh) {
   memset(t.data(), 0, (E + 1) * sizeof(RbtExpertDev));
   int kind = -1;
   size_t gs = 0;
+  bool al = true;
   for (auto it = c->pool.lower_bound((uint64_t)layer << 32); it != c->pool.end() && (uint32_t)(it->first >> 32) == layer;
        ++it) {
     const uint32_t eid = (uint32_t)it->first;
@@ -513,6 +599,7 @@ int refresh_latent(rbt_ctx *c, uint32_t layer, Layer &L, size_t mh) {
     if (kind >= 0 && (kd != kind || g != gs)) return fail(c, RBT_E_UNSUPPORTED, "layer %u: experts mix formats", layer);
     kind = kd;
     gs = g;
+    al = al && al16(t[eid]);
   }
   if (kind < 0) return fail(c, RBT_E_NOT_RESIDENT, "layer %u has no resident experts", layer);
   if (L.lat_cap < E + 1) {
@@ -526,6 +613,7 @@ int refresh_latent(rbt_ctx *c, uint32_t layer, Layer &L, size_t mh) {
   HIP_OK(c, hipStreamSynchronize(c->stream));
   L.lat_kind = kind;
   L.lat_gs = gs;
+  L.lat_al16 = al;
   L.lat_mh = mh;
   L.lat_dirty = false;
   return RBT_OK;
@@ -738,6 +826,86 @@ int decode_grouped_dev(rbt_ctx *c, Layer &L, const float *x, int S, int k, int E
   return RBT_OK;
 }
 
+// A batch's grouped scratch: [bits E W][pc E W][segs][tiles][ntiles].
+size_t group_scratch(int S, int E, long max_tiles, size_t (&off)[4]) {
+  const size_t W = (S + 31) / 32;
+  off[0] = align256((size_t)E * W * 4);
+  off[1] = off[0] + align256((size_t)E * W * 4);
+  off[2] = off[1] + align256(sizeof(rbt::PSeg) * rbt::PG_MAXE);
+  off[3] = off[2] + align256(sizeof(rbt::PTile) * (size_t)max_tiles);
+  return off[3] + 256;
+}
+
+bool x3_experts_ok(rbt_ctx *c, int kind, size_t gs, bool aligned, const float *x, int S, int k, int E, int H, int I,
+                   int has_shared) {
+  size_t off[4];
+  // The tiled products stream each unique expert once, the GEMVs once per (token, expert) pair and
+  // somewhat faster. int4, hidden 6144, top-8 of 256 and a shared expert, us, GEMV against tiled: 4 tokens
+  // 197 / 203, 6 271 / 289, 8 345 / 333, 16 650 / 572, 40 1553 / 952: the line lies where the pairs are
+  // 1.22 times the experts that uniform routing picks.
+  const double uniq = E * (1.0 - std::pow(1.0 - std::min(1.0, (double)k / E), S)) + has_shared;
+  return S >= 2 && (double)S * (k + has_shared) >= 1.22 * uniq && aligned && al16({x}) && (size_t)6 * S * H < ((size_t)1 << 32) &&
+         rbt::x3_ok(kind, gs, H, I, true) &&
+         rbt::x3_ok(kind, gs, I, H, false) && E + 1 <= rbt::PG_MAXE &&
+         scratch_avail(c, {{SC_PGRP, group_scratch(S, E, rbt::x3_max_tiles(S, k, E, has_shared, 16), off)},
+                           {SC_XB, (size_t)6 * S * H}});
+}
+
+// A batch through its routed (and shared) experts with fp32 accuracy, every unique expert's weights
+// streamed once per tile of its tokens: grouping, the activations' exact parts, gate/up with the
+// activation, down. yy [pairs, H] gets the pairs' rows in launch_pgroup's order, tpair / tw what
+// launch_combine needs. h: 2 I floats per pair.
+int x3_experts(rbt_ctx *c, int kind, const RbtExpertDev *table, const RbtExpertDev *shared_dev, int has_shared,
+               const float *x, int S, int k, int E, int H, int I, const int32_t *ids, const float *wts, int *ptok,
+               int *tpair, float *tw, float *h, float *yy, const RbtAct &act, hipEvent_t *ev) {
+  const int tch = x3_tch((size_t)S * k / E);
+  size_t off[4];
+  void *blk;
+  RBT_TRY(scratch(c, SC_PGRP, group_scratch(S, E, rbt::x3_max_tiles(S, k, E, has_shared, 16), off), &blk));
+  char *b = static_cast<char *>(blk);
+  rbt::PSeg *segs = reinterpret_cast<rbt::PSeg *>(b + off[1]);
+  rbt::PTile *tiles = reinterpret_cast<rbt::PTile *>(b + off[2]);
+  int *ntiles = reinterpret_cast<int *>(b + off[3]);
+  __bf16 *xb3;
+  RBT_TRY(scratch_t(c, SC_XB, (size_t)3 * S * H, &xb3));
+  int *dflags = c->d_flags;
+  HIP_OK(c, rbt::launch_pgroup(*c, ids, wts, S, k, E, has_shared, table, reinterpret_cast<uint32_t *>(b),
+                               reinterpret_cast<uint32_t *>(b + off[0]), segs, tiles, ntiles, ptok, tpair, tw,
+                               dflags + FLAG_ERR, dflags + FLAG_UNIQ, tch));
+  HIP_OK(c, rbt::launch_x3split(*c, kind, x, S, H, xb3, c->d_queue));
+  rbt::X3Args A;
+  A.tch = tch;
+  A.tiles = tiles;
+  A.ntiles = ntiles;
+  A.segs = segs;
+  A.table = table;
+  A.shared_dev = shared_dev;
+  A.row_tok = ptok;
+  A.S = S;
+  A.xb3 = xb3;
+  A.K = H;
+  A.O = I;
+  A.hb3 = reinterpret_cast<__bf16 *>(h);  // [3 pairs, I]
+  A.act = act;
+  A.queue = c->d_queue;
+  if (ev) HIP_OK(c, hipEventRecord(ev[1], c->stream));
+  if (ev) c->t_start = ev[2], c->t_stop = ev[3];
+  const hipError_t e1 = rbt::launch_x3(*c, kind, true, A);
+  c->t_start = c->t_stop = nullptr;
+  HIP_OK(c, e1);
+  A.row_tok = nullptr;
+  A.xb3 = A.hb3;
+  A.K = I;
+  A.O = H;
+  A.y = yy;
+  A.queue = c->d_queue + 8;
+  if (ev) c->t_start = ev[4], c->t_stop = ev[5];
+  const hipError_t e2 = rbt::launch_x3(*c, kind, false, A);
+  c->t_start = c->t_stop = nullptr;
+  HIP_OK(c, e2);
+  return RBT_OK;
+}
+
 // accumulate: out += the layer's output (x and out must not overlap). The one-token down launch adds
 // in its own store; the other paths write the output to a scratch and add it after.
 // norm_w (the MoE sublayer): the layer's input is rmsnorm_1p(x, norm_w, eps) (qwen38/ops.rs:25-33),
@@ -911,7 +1079,13 @@ int moe_forward_dev(rbt_ctx *c, uint32_t layer, const float *x, size_t s, float 
   }
   const bool grouped = !dgrouped && !mfma && S > 1 && (merge || !D.has_shared) &&
                        rbt::prefill_ok(L.routed_kind, H, I, (size_t)E, (size_t)k);
-  if (dgrouped) {
+  const bool x3 = !dgrouped && !grouped && !mfma && (merge || !D.has_shared) &&
+                  x3_experts_ok(c, L.routed_kind, L.routed_gs, L.al16, x, S, k, E, H, I, D.has_shared ? 1 : 0);
+  if (x3) {
+    RBT_TRY(x3_experts(c, L.routed_kind, L.d_table, L.d_shared, D.has_shared ? 1 : 0, x, S, k, E, H, I, ids, wts, ptok,
+                       tpair, tw, h, yy, RbtAct{}, c->prof ? ev.data() : nullptr));
+    HIP_OK(c, rbt::launch_combine(*c, yy, S, k, H, tpair, tw, shs, D.has_shared, gated, dst));
+  } else if (dgrouped) {
     RBT_TRY(decode_grouped_dev(c, L, x, S, k, E, H, I, ids, wts, shs, ptok, tpair, tw, h, yy, gated, dst,
                                c->prof ? ev.data() : nullptr, xb3_sel));
   } else if (grouped) {
@@ -1243,9 +1417,10 @@ int rbt_init(rbt_ctx **out, int device) {
     c->num_cu = prop.multiProcessorCount;
   const char *what = nullptr;
   if ((e = hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking)) != hipSuccess) what = "hipStreamCreateWithFlags";
-  else if ((e = hipMalloc((void **)&c->d_flags, (FLAG_N + rbt::CNT_N) * sizeof(int))) != hipSuccess) what = "hipMalloc";
-  else if ((e = hipMemset(c->d_flags, 0, (FLAG_N + rbt::CNT_N) * sizeof(int))) != hipSuccess) what = "hipMemset";
+  else if ((e = hipMalloc((void **)&c->d_flags, (FLAG_N + rbt::CNT_N + rbt::X3_QN) * sizeof(int))) != hipSuccess) what = "hipMalloc";
+  else if ((e = hipMemset(c->d_flags, 0, (FLAG_N + rbt::CNT_N + rbt::X3_QN) * sizeof(int))) != hipSuccess) what = "hipMemset";
   if (!what) c->d_cnt = reinterpret_cast<unsigned *>(c->d_flags + FLAG_N);
+  if (!what) c->d_queue = c->d_cnt + rbt::CNT_N;
   // the allocation-free entry point's scratch on this device (the device is current)
   if (!what) c->noalloc = noalloc_base(device, &c->noalloc_err);
   if (what) {

@@ -26,6 +26,7 @@ struct Ctx {
   // Arrival counters (CNT_N, device memory, zeroed at creation): a kernel that counts arrivals on
   // them returns each to 0 before it ends.
   unsigned *d_cnt = nullptr;
+  unsigned *d_queue = nullptr;  // unit queues (X3_QN, device memory), cleared by the launch before their use
 };
 constexpr int CNT_N = 1024;
 
@@ -199,6 +200,45 @@ hipError_t launch_pgateup(const Ctx &c, const PTile *tiles, const int *ntiles, l
 hipError_t launch_pdown(const Ctx &c, const PTile *tiles, const int *ntiles, long max_tiles, const PSeg *segs,
                         const RbtExpertDev *table, const RbtExpertDev *shared_dev, const __bf16 *hb, int I, int H,
                         float *y);
+
+// x3gemm.hip: batches with fp32 accuracy on the matrix cores (three exact bf16 parts per activation),
+// MXFP4 or grouped int4 (groups of 32). Rows are tiled by tch (16 or 32); with tiles (launch_pgroup,
+// the same tch) the call is grouped over experts, else `single` takes rows 0 .. min(nrows, *nrows_dev)
+// - 1.
+struct X3Args {
+  const PTile *tiles = nullptr;
+  const int *ntiles = nullptr;
+  const PSeg *segs = nullptr;
+  const RbtExpertDev *table = nullptr, *shared_dev = nullptr;
+  RbtExpertDev single{};
+  const int *nrows_dev = nullptr;
+  int nrows = 0;
+  const int *row_tok = nullptr;  // activation row of pair p (null: p), below S
+  int S = 0;
+  const __bf16 *xb3 = nullptr;  // [3 rows, K] parts
+  int tch = 16;                 // rows per tile
+  int K = 0, O = 0;             // columns, rows of one matrix
+  int KS = 1;                   // K parts (single only): y takes [KS][matrices][nrows, O] partial sums
+  __bf16 *hb3 = nullptr;        // gate/up, KS = 1: act(g, u) as the down product's parts [3 pairs, O]
+  float *y = nullptr;           // down / matrix: [pairs, O]
+  RbtAct act{};
+  unsigned *queue = nullptr;  // grouped: 8 cleared counters, units are taken in turn
+};
+constexpr int X3_QN = 16;
+// gateup: gate and up with the activation (64-row blocks); else one matrix (128-row blocks).
+bool x3_ok(int kind, size_t gs, size_t cols, size_t rows, bool gateup);
+// Tiles of launch_pgroup over S tokens, at most.
+long x3_max_tiles(int S, int k, int E, int has_shared, int tch);
+// K parts that fill the chip for n rows through one matrix (or one expert's gate and up).
+int x3_parts(const Ctx &c, size_t n, int tch, size_t cols, size_t rows, bool gateup);
+// x and xb3 16-byte aligned, K a multiple of 8. queue: X3_QN counters to clear (8 per product).
+hipError_t launch_x3split(const Ctx &c, int kind, const float *x, size_t S, size_t K, __bf16 *xb3,
+                          unsigned *queue = nullptr);
+hipError_t launch_x3(const Ctx &c, int kind, bool gateup, const X3Args &A);
+// After launch_x3 with KS > 1: y[n] = the sum of the KS partial vectors (n a multiple of 4), or (gate/
+// up) A.hb3 from the partial sums in A.y.
+hipError_t launch_x3sum(const Ctx &c, const float *part, size_t n, int KS, float *y);
+hipError_t launch_x3act(const Ctx &c, int kind, const X3Args &A);
 
 // router.hip
 hipError_t launch_router_logits(const Ctx &c, const float *x, int S, int H, const float *W, int E, const float *sgate,

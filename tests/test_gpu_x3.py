@@ -1,0 +1,88 @@
+"""Batches through the tiled matrix-core products (x3gemm.hip), at the sizes where they can go wrong: the
+edges of the token tiles (5, 16 and 32 tokens), one and several 512-column groups, K parts that do not
+divide the columns evenly, a number of row blocks that is no multiple of anything.
+
+Bar: 1e-6 relative 2-norm against a 64-bit product of the dequantized weights. The products are exact and
+a row's sum is at most 48 MFMA roundings per 256 columns and one addition per 32 (int4) or 256 (MXFP4)
+columns: rounding errors u = 2^-24 at random signs give u sqrt(n / 6) with n <= 256, about 4e-7.
+"""
+import numpy as np
+import pytest
+
+from helpers import HipGraph, normal, rel_l2
+from test_gpu_moe import _small_layer
+
+pytestmark = pytest.mark.gpu
+
+
+def _matrix(ctx, orc, fmt, rows, cols, seed):
+    import torch
+    import rabbit_amd as R
+    q = orc.synth_mxfp4(rows, cols, seed) if fmt == "mxfp4" else orc.synth_i4g(rows, cols, 32, seed)
+    data, scale = torch.from_numpy(q.data).cuda(), torch.from_numpy(q.scale).cuda()
+    w = R.QT.mxfp4(data, scale, rows, cols) if fmt == "mxfp4" else R.QT.i4g(data, scale, rows, cols, 32)
+    return w, ctx.dequant_rows(w, 0, rows).reshape(rows, cols).double()
+
+
+# tokens * columns * rows past the line where the tiled products take over; (2048, 1152): the GEMV below it
+@pytest.mark.parametrize("fmt", ["mxfp4", "i4g"])
+@pytest.mark.parametrize("cols,rows,tokens", [(7168, 3584, (2, 4, 5, 6, 16, 17, 33)), (512, 16512, (12, 32, 49)),
+                                              (2048, 1152, (21, 22, 43, 48, 130)), (4608, 640, (34, 64, 65))])
+def test_matmul_batches(ctx, orc, fmt, cols, rows, tokens):
+    import torch
+    w, dense = _matrix(ctx, orc, fmt, rows, cols, cols + rows)
+    for s in tokens:
+        x = torch.from_numpy(normal((s, cols), s)).cuda()
+        y = torch.full((s + 1, rows), 7.0, device="cuda")
+        ctx.matmul_qt(y[:s], x, w, s)
+        err = float((y[:s].double() - x.double() @ dense.t()).norm() / (x.double() @ dense.t()).norm())
+        assert err < 1e-6, (s, err)
+        assert bool((y[s] == 7.0).all()), s  # nothing past the last token
+
+
+@pytest.mark.parametrize("E,k,S", [(24, 4, 40), (24, 4, 61), (3, 2, 37), (2, 1, 70), (6, 6, 2)])
+def test_int4_layer_batches(ctx, orc, E, k, S):
+    """Grouped int4 layers whose experts take 1..5, 6..16 and 17..32 tokens, with the shared expert's tiles."""
+    import rabbit_amd as R
+    H, I = 512, 512
+    L = _small_layer(ctx, orc, 1, R.QT_I4_GROUPED, H, I, E, k, seed=E + S)
+    x = normal((S, H), S)
+    exp, eids, _ = L.forward(x, S)
+    out, ids, w = np.empty(S * H, np.float32), np.empty(S * k, np.int32), np.empty(S * k, np.float32)
+    ctx.moe_forward(0, x, S, out, ids, w)
+    assert np.array_equal(ids.reshape(S, k), eids)
+    for t in range(S):
+        assert rel_l2(out[t * H:(t + 1) * H], np.asarray(exp).reshape(S, H)[t]) < 1e-5, t
+
+
+def test_captured_batches(rbt_lib, orc):
+    """A batch captured on a context that never ran one (no scratch to be had inside the capture: the GEMV
+    path, which needs none) and captured again after an eager call: every replay equals an eager call."""
+    import torch
+    import rabbit_amd as R
+    ctx = R.Context(0)
+    rows, cols, s = 3584, 7168, 9
+    w, dense = _matrix(ctx, orc, "i4g", rows, cols, 3)
+    x = torch.empty(s, cols, device="cuda")
+    y = torch.empty(s, rows, device="cuda")
+    q = w.c()
+    import ctypes as C
+    for _ in range(2):
+        g = HipGraph(ctx.stream)
+        torch.cuda.synchronize()
+        g.begin()
+        rc = ctx.lib.rbt_matmul_qt_d(ctx.h, y.data_ptr(), x.data_ptr(), C.byref(q), s)
+        g.end()
+        assert rc == 0
+        for i in range(3):
+            x.copy_(torch.from_numpy(normal((s, cols), 50 + i)))
+            torch.cuda.synchronize()
+            g.launch()
+            ctx.sync()
+            want = x.double() @ dense.t()
+            assert float((y.double() - want).norm() / want.norm()) < 1e-6
+            ye = torch.empty_like(y)
+            ctx.matmul_qt(ye, x, w, s)
+            assert float((y - ye).norm() / ye.norm()) < 1e-6
+        g.destroy()
+    ctx.close()
