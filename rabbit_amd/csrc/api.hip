@@ -429,10 +429,10 @@ const PoolEntry *find_pool_slot(rbt_ctx *c, const rbt_expert_slot *s) {
 
 // Whether a batch through one matrix takes the tiled matrix-core kernels (split, product, sum of the K
 // parts: about 14 us of launches) rather than the GEMV per token, whose time grows with s. us, GEMV
-// against tiled: int4 7168 x 3584 s = 2 19.3 / 16.7, 16 63.6 / 20.5, 512 1615 / 135; MXFP4 3584 x 3072
+// against tiled: int4 7168 x 3584 s = 2 19.3 / 16.7, 3 25.2 / 16.9, 16 63.6 / 20.5, 512 1615 / 135; MXFP4 3584 x 3072
 // s = 4 9.7 / 14.3, 16 18.7 / 14.2, 64 55.5 / 21.2; 2048 x 8192 s = 4 10.0 / 14.0, 16 24.4 / 13.8.
 bool x3_matmul_wins(int kind, size_t s, size_t i, size_t o) {
-  return s >= 2 && s * i * o >= (size_t)(kind == RBT_QT_I4_GROUPED ? 50 : 100) * 1000000;
+  return s >= 2 && s * i * o >= (size_t)(kind == RBT_QT_I4_GROUPED ? 75 : 100) * 1000000;
 }
 
 // Rows per tile: 32 where the rows of one matrix (or an expert, on average) go past 16.
@@ -842,9 +842,10 @@ bool x3_experts_ok(rbt_ctx *c, int kind, size_t gs, bool aligned, const float *x
   // The tiled products stream each unique expert once, the GEMVs once per (token, expert) pair and
   // somewhat faster. int4, hidden 6144, top-8 of 256 and a shared expert, us, GEMV against tiled: 4 tokens
   // 197 / 203, 6 271 / 289, 8 345 / 333, 16 650 / 572, 40 1553 / 952: the line lies where the pairs are
-  // 1.22 times the experts that uniform routing picks.
+  // 1.22 times the experts that uniform routing picks. MXFP4 (moe_hidden 3584 x 3072, top-16 of 896):
+  // 4 tokens 320 / 336, 8 552 / 514, 16 970 / 834, 131 6.9 ms / 2.5 ms: 1.06 times.
   const double uniq = E * (1.0 - std::pow(1.0 - std::min(1.0, (double)k / E), S)) + has_shared;
-  return S >= 2 && (double)S * (k + has_shared) >= 1.22 * uniq && aligned && al16({x}) && (size_t)6 * S * H < ((size_t)1 << 32) &&
+  return S >= 2 && (double)S * (k + has_shared) >= (kind == RBT_QT_I4_GROUPED ? 1.22 : 1.06) * uniq && aligned && al16({x}) && (size_t)6 * S * H < ((size_t)1 << 32) &&
          rbt::x3_ok(kind, gs, H, I, true) &&
          rbt::x3_ok(kind, gs, I, H, false) && E + 1 <= rbt::PG_MAXE &&
          scratch_avail(c, {{SC_PGRP, group_scratch(S, E, rbt::x3_max_tiles(S, k, E, has_shared, 16), off)},
@@ -903,6 +904,37 @@ int x3_experts(rbt_ctx *c, int kind, const RbtExpertDev *table, const RbtExpertD
   const hipError_t e2 = rbt::launch_x3(*c, kind, false, A);
   c->t_start = c->t_stop = nullptr;
   HIP_OK(c, e2);
+  return RBT_OK;
+}
+
+// Router logits and selection of a call (not the one-token fused launches): a decode batch as certified
+// intervals for every (row, token) with a selection workgroup per token (whose idle waves write xb3_sel,
+// the tokens' three-part split, when given); larger batches on the matrix cores with a rigorous bound on
+// the distance to the reference's sequential fp32 fold, or as that fold itself.
+int route_logits_select(rbt_ctx *c, const rbt::RouterArgs &ra, int erows, const float *sgate, const RbtExpertDev *table,
+                        double *mid, double *bnd, int32_t *ids, float *wts, float *shs, const rbt::GroupArgs *ga,
+                        const rbt::SharedGateUp *sgu, __bf16 *xb3_sel) {
+  int *amb = c->d_flags + FLAG_AMB;
+  const bool al = al16({ra.x, ra.W, sgate});
+  const bool bounded = ra.S >= rbt::RB_MIN_S && rbt::router_bounded_ok(ra) && al &&
+                       (ra.S >= 64 || scratch_avail(c, {{SC_RLOG, rbt::router_bounded_scratch(ra, erows)}}));
+  if (!bounded && !rbt::router_exact_ok(ra.S, ra.H) && rbt::router_batch_ok(ra) && al16({sgate})) {
+    HIP_OK(c, rbt::launch_router_batch(*c, ra, sgate, mid, bnd, table, ids, wts, shs, amb, xb3_sel));
+    return RBT_OK;
+  }
+  if (bounded) {
+    void *rs;
+    RBT_TRY(scratch(c, SC_RLOG, rbt::router_bounded_scratch(ra, erows), &rs));
+    HIP_OK(c, rbt::launch_router_bounded(*c, ra, sgate, mid, bnd, rs));
+  } else if (rbt::router_exact_ok(ra.S, ra.H) && al) {
+    float *lg;
+    RBT_TRY(scratch_t(c, SC_RLOG, (size_t)ra.S * erows, &lg));
+    HIP_OK(c, rbt::launch_router_logits_exact(*c, ra.x, ra.S, ra.H, ra.W, ra.E, sgate, lg));
+    HIP_OK(c, rbt::launch_logits_to_mid(*c, lg, (size_t)ra.S * erows, mid, bnd));
+  } else {
+    HIP_OK(c, rbt::launch_router_logits(*c, ra.x, ra.S, ra.H, ra.W, ra.E, sgate, mid, bnd));
+  }
+  HIP_OK(c, rbt::launch_router_select(*c, ra, mid, bnd, ids, wts, shs, amb, ga, sgu));
   return RBT_OK;
 }
 
@@ -1052,30 +1084,12 @@ int moe_forward_dev(rbt_ctx *c, uint32_t layer, const float *x, size_t s, float 
     if (fold_norm) rr.x = xraw;
     HIP_OK(c, rbt::launch_router1(*c, rr, sgate, mid, bnd, shs, rec, fold_norm ? norm_w : nullptr, eps,
                                   fold_norm ? xn : nullptr));
-  } else if (!rbt::router_exact_ok(S, H) && rbt::router_batch_ok(ra) && (uintptr_t)(sgate ? sgate : x) % 16 == 0) {
-    // a decode batch: certified intervals for every (row, token), then the per-token selection (whose
-    // idle waves split the tokens for the grouped decode GEMMs)
-    if (dgrouped && (uintptr_t)x % 16 == 0 && H % 4 == 0) RBT_TRY(scratch_t(c, SC_XB, (size_t)3 * S * H, &xb3_sel));
-    HIP_OK(c, rbt::launch_router_batch(*c, ra, sgate, mid, bnd, L.d_table, ids, wts, shs, dflags + FLAG_AMB, xb3_sel));
   } else {
-    const bool al16 = ((uintptr_t)x | (uintptr_t)D.router | (uintptr_t)(sgate ? sgate : x)) % 16 == 0;
-    if (rbt::router_exact_ok(S, H) && rbt::router_bounded_ok(ra) && al16) {
-      // batches: fp64-accurate logits on the matrix cores with a rigorous bound on their distance to
-      // the reference's sequential fp32 fold (the selection folds the ambiguous experts exactly)
-      void *rs;
-      RBT_TRY(scratch(c, SC_RLOG, rbt::router_bounded_scratch(ra, erows), &rs));
-      HIP_OK(c, rbt::launch_router_bounded(*c, ra, sgate, mid, bnd, rs));
-    } else if (rbt::router_exact_ok(S, H) && al16) {
-      // batches: the reference's sequential fp32 logits themselves, then point intervals
-      float *lg;
-      RBT_TRY(scratch_t(c, SC_RLOG, (size_t)S * erows, &lg));
-      HIP_OK(c, rbt::launch_router_logits_exact(*c, x, S, H, D.router, E, sgate, lg));
-      HIP_OK(c, rbt::launch_logits_to_mid(*c, lg, (size_t)S * erows, mid, bnd));
-    } else {
-      HIP_OK(c, rbt::launch_router_logits(*c, x, S, H, D.router, E, sgate, mid, bnd));
-    }
-    HIP_OK(c, rbt::launch_router_select(*c, ra, mid, bnd, ids, wts, shs, dflags + FLAG_AMB,
-                                        grp_in_select ? &ga : nullptr, sh_in_select ? &sgu : nullptr));
+    // the batch selection's idle waves split the tokens for the grouped decode GEMMs
+    if (dgrouped && !rbt::router_exact_ok(S, H) && rbt::router_batch_ok(ra) && al16({sgate, x}) && H % 4 == 0)
+      RBT_TRY(scratch_t(c, SC_XB, (size_t)3 * S * H, &xb3_sel));
+    RBT_TRY(route_logits_select(c, ra, erows, sgate, L.d_table, mid, bnd, ids, wts, shs, grp_in_select ? &ga : nullptr,
+                                sh_in_select ? &sgu : nullptr, xb3_sel));
   }
   const bool grouped = !dgrouped && !mfma && S > 1 && (merge || !D.has_shared) &&
                        rbt::prefill_ok(L.routed_kind, H, I, (size_t)E, (size_t)k);
@@ -1319,14 +1333,6 @@ static int latent_moe_dev(rbt_ctx *c, uint32_t layer, const rbt_latent_moe_desc 
                                    (int)MH, yy, (long)MH));
     }
   } else {
-  if (rbt::router_exact_ok(S, (int)H) && ((uintptr_t)x | (uintptr_t)D.router) % 16 == 0) {
-    float *lg;
-    RBT_TRY(scratch_t(c, SC_RLOG, (size_t)S * E, &lg));
-    HIP_OK(c, rbt::launch_router_logits_exact(*c, x, S, (int)H, D.router, (int)E, nullptr, lg));
-    HIP_OK(c, rbt::launch_logits_to_mid(*c, lg, (size_t)S * E, mid, bnd));
-  } else {
-    HIP_OK(c, rbt::launch_router_logits(*c, x, S, (int)H, D.router, (int)E, nullptr, mid, bnd));
-  }
   // one token: the selection writes the pair list itself (pair j = slot j)
   const bool grp_in_select = S == 1 && !(D.n_group > 1 && D.family != RBT_FAMILY_QWEN38);
   rbt::GroupArgs ga{table, table + E, pjob, ptok, tpair, tw, dflags + FLAG_ERR};
@@ -1334,20 +1340,26 @@ static int latent_moe_dev(rbt_ctx *c, uint32_t layer, const rbt_latent_moe_desc 
   if (dp_fused) {
     // one token: the latent down projection streams while the selection runs (one launch)
     RBT_TRY(check_qt(c, &Dp, "matmul"));
+    HIP_OK(c, rbt::launch_router_logits(*c, x, S, (int)H, D.router, (int)E, nullptr, mid, bnd));
     RbtExpertDev pj{};
     pj.dd = (const uint8_t *)Dp.data;
     pj.ds = Dp.scale;
     HIP_OK(c, rbt::launch_router_select_dp(*c, ra, mid, bnd, ids, wts, shs, dflags + FLAG_AMB, ga, pj, Dp.kind,
                                            (int)H, (int)MH, xl));
   } else {
-    HIP_OK(c, rbt::launch_router_select(*c, ra, mid, bnd, ids, wts, shs, dflags + FLAG_AMB,
-                                        grp_in_select ? &ga : nullptr));
+    RBT_TRY(route_logits_select(c, ra, (int)E, nullptr, table, mid, bnd, ids, wts, shs, grp_in_select ? &ga : nullptr,
+                                nullptr, nullptr));
     RBT_TRY(matmul_dev(c, xl, x, &lw->down_proj, s));
   }
-  if (!grp_in_select)
-    HIP_OK(c, rbt::launch_group(*c, ids, wts, S, K, (int)E, table, table + E, pjob, ptok, tpair, tw,
-                                dflags + FLAG_ERR, dflags + FLAG_UNIQ));
-  RBT_TRY(expert_pairs(c, kind, gs, pjob, none, P, nullptr, xl, ptok, MH, I, h, yy, nullptr, act));
+  if (x3_experts_ok(c, kind, gs, Ly.lat_al16, xl, S, K, (int)E, (int)MH, (int)I, 0)) {
+    RBT_TRY(x3_experts(c, kind, table, table + E, 0, xl, S, K, (int)E, (int)MH, (int)I, ids, wts, ptok, tpair, tw, h,
+                       yy, act, nullptr));
+  } else {
+    if (!grp_in_select)
+      HIP_OK(c, rbt::launch_group(*c, ids, wts, S, K, (int)E, table, table + E, pjob, ptok, tpair, tw,
+                                  dflags + FLAG_ERR, dflags + FLAG_UNIQ));
+    RBT_TRY(expert_pairs(c, kind, gs, pjob, none, P, nullptr, xl, ptok, MH, I, h, yy, nullptr, act));
+  }
   }
   if (!combined) HIP_OK(c, rbt::launch_combine(*c, yy, S, K, (int)MH, tpair, tw, shs, 0, 0, routed));
   const rbt_qt &U = lw->up_proj;
@@ -1358,6 +1370,7 @@ static int latent_moe_dev(rbt_ctx *c, uint32_t layer, const rbt_latent_moe_desc 
     HIP_OK(c, rbt::launch_proj1(*c, U.kind, U.group_size, U.data, U.scale, routed, (int)MH, (int)H, out, lw->norm,
                                 lw->eps));
   } else if (lw->norm && U.kind != RBT_QT_F32 && rbt::decode_shape_ok(MH, U.kind, U.group_size) &&
+      !x3_matmul_wins(U.kind, s, MH, H) &&
       ((uintptr_t)U.data | (uintptr_t)lw->norm) % 16 == 0) {
     // the norm of each summed row inside the up projection's waves, which read the whole row
     RBT_TRY(check_qt(c, &U, "matmul"));

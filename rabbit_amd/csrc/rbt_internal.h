@@ -358,6 +358,7 @@ hipError_t launch_logits_to_mid(const Ctx &c, const float *logits, size_t n, dou
 // Batched router logits on the matrix cores, certified: mid (fp64-accurate) and a rigorous bound on
 // the distance to the reference's sequential fp32 fold, for launch_router_select (which folds the
 // ambiguous ones exactly). scratch: router_bounded_scratch bytes.
+constexpr int RB_MIN_S = 17;
 bool router_bounded_ok(const RouterArgs &a);
 size_t router_bounded_scratch(const RouterArgs &a, int erows);
 hipError_t launch_router_bounded(const Ctx &c, const RouterArgs &a, const float *sgate, double *mid, double *bnd,

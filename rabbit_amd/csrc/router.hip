@@ -2899,6 +2899,9 @@ hipError_t launch_router_batch(const Ctx &c, const RouterArgs &a, const float *s
   const SelParams P = sel_params(a);
   launch_k(c, k_router_logits_t1, dim3(a.erows, a.S), dim3(256), a.x, a.S, a.H, a.W, a.E, sgate, mid, bnd, a.erows);
   const int m = (a.E + 63) / 64;
+  // past 512 experts one wave's record selection is slower than the whole-workgroup one (896 experts:
+  // 55 us against 47 for 2 tokens, 62 against 54 for 40)
+  if (m > 8 && !xb3) return launch_router_select(c, a, mid, bnd, ids, wts, sh_scale, stats);
   if (m <= 4)
     launch_k(c, k_router_select_rec<4>, dim3(a.S), dim3(256), P, (const double *)mid, (const double *)bnd, table, ids,
              wts, sh_scale, stats, xb3);

@@ -86,3 +86,16 @@ def test_captured_batches(rbt_lib, orc):
             assert float((y - ye).norm() / ye.norm()) < 1e-6
         g.destroy()
     ctx.close()
+
+
+# 600 experts: the batch selection past 512; 24 experts of 3 to 40 tokens: every tile form with Situ
+@pytest.mark.parametrize("E,k,S", [(600, 4, 2), (600, 4, 40), (24, 4, 11), (24, 4, 60), (6, 4, 66)])
+def test_latent_batches(ctx, orc, E, k, S):
+    import rabbit_amd as R
+    from test_gpu_latent import _latent_case, _run_latent
+    H, MH, I = 1024, 512, 512 if E < 600 else 64
+    layer = 70 + E % 7
+    L, dq, uq, _ = _latent_case(ctx, orc, layer, H, MH, I, E, k, 4000 + E, "i4g", 1.0)
+    x = normal((S, H), S, 1.0)
+    norm = np.abs(normal(MH, 5, 1.0)) + np.float32(0.5)
+    _run_latent(ctx, R, layer, L, dq, uq, x, S, MH, norm, orc.situ(4.0, 25.0), R.situ(4.0, 25.0))
