@@ -443,8 +443,9 @@ int x3_tch(size_t rows) { return rows > 16 ? 32 : 16; }
 // needs cannot be had (the caller takes another path).
 int x3_matmul(rbt_ctx *c, float *y, const float *x, const rbt_qt *w, size_t s) {
   const size_t i = w->cols, o = w->rows;
-  // the partial sums' bound over every s up to this one, so that a smaller batch never grows it
-  const size_t part = (64 * (size_t)c->num_cu / (o / 128) + s + 32) * o;
+  // (a bound over every s up to this one, so that a smaller batch never grows it)
+  const int rb = rbt::x3_row_blocks((int)o, false);
+  const size_t part = rbt::x3_part_rows(*c, s, rb) * o;
   if (!scratch_avail(c, {{SC_XB, 6 * s * i}, {SC_XP, 4 * part}})) return 1;
   __bf16 *xb3;
   float *xp;
@@ -458,11 +459,13 @@ int x3_matmul(rbt_ctx *c, float *y, const float *x, const rbt_qt *w, size_t s) {
   A.K = (int)i;
   A.O = (int)o;
   A.tch = x3_tch(s);
-  A.KS = rbt::x3_parts(*c, s, A.tch, i, o, false);
-  A.y = A.KS > 1 ? xp : y;
+  A.wgs = rbt::x3_wgs(*c, A.tch);
+  const int ks = rbt::x3_ks((long)s, A.tch, (int)i, rb, A.wgs);
+  A.part = ks > 1;
+  A.y = A.part ? xp : y;
   HIP_OK(c, rbt::launch_x3split(*c, w->kind, x, s, i, xb3));
   HIP_OK(c, rbt::launch_x3(*c, w->kind, false, A));
-  if (A.KS > 1) HIP_OK(c, rbt::launch_x3sum(*c, xp, s * o, A.KS, y));
+  if (A.part) HIP_OK(c, rbt::launch_x3sum(*c, xp, s * o, ks, y));
   return RBT_OK;
 }
 
@@ -1209,6 +1212,12 @@ int to_act(rbt_ctx *c, const rbt_activation *a, RbtAct *out) {
   return RBT_OK;
 }
 
+// Tokens from which one expert's batch takes the tiled products (five launches, about 28 us) rather than
+// GEMVs per token that picked it. Half of the tokens picking, us, GEMV against tiled: MXFP4 8192 x 2048
+// 4 tokens 29.2 / 28.4, 8 37.1 / 29.4, 64 170 / 45, 256 633 / 76; int4 4 tokens 31.0 / 29.9, 8 41.4 / 30.5,
+// 256 780 / 86.
+bool x3_expert_wins(size_t s) { return s >= 5; }
+
 int apply_single_dev(rbt_ctx *c, const rbt_expert_slot *slot, const int32_t *ids, const float *w, size_t s, size_t k,
                      const float *x, size_t d, size_t i, const RbtAct &act, float *out) {
   if (!slot || !ids || !w || !x || !out) return fail(c, RBT_E_INVALID, "null argument");
@@ -1226,6 +1235,50 @@ int apply_single_dev(rbt_ctx *c, const rbt_expert_slot *slot, const int32_t *ids
     HIP_OK(c, rbt::launch_xexpert1(*c, v, x, (int)d, (int)i, ids, w, (int)k, (int)slot->eid,
                                    reinterpret_cast<__bf16 *>(hs), out, act));
     return RBT_OK;
+  }
+  const int rbg = rbt::x3_row_blocks((int)i, true), rbd = rbt::x3_row_blocks((int)d, false);
+  if (x3_expert_wins(s) && 6 * s * std::max(d, i) < ((size_t)1 << 32) && al16({x, out}) && al16(v) &&
+      rbt::x3_ok(kind, gs, d, i, true) && rbt::x3_ok(kind, gs, i, d, false)) {
+    // a batch: the tiled products over the tokens that picked the expert (their number on the device), K
+    // split by what it leaves idle. Partial sums' bounds hold for every s up to this one.
+    const size_t pg = rbt::x3_part_rows(*c, s, rbg) * 2 * i, pd = rbt::x3_part_rows(*c, s, rbd) * d;
+    if (scratch_avail(c, {{SC_XB, 6 * s * d}, {SC_H, 6 * s * i}, {SC_XP, 4 * std::max(pg, pd)}, {SC_PTOK, 4 * s},
+                          {SC_TW, 4 * s}, {SC_FLAGS, 16}})) {
+      __bf16 *xb3, *hb3;
+      float *xp, *pw;
+      int *ptok, *nr;
+      RBT_TRY(scratch_t(c, SC_XB, 3 * s * d, &xb3));
+      RBT_TRY(scratch_t(c, SC_H, 3 * s * i, &hb3));
+      RBT_TRY(scratch_t(c, SC_XP, std::max(pg, pd), &xp));
+      RBT_TRY(scratch_t(c, SC_PTOK, s, &ptok));
+      RBT_TRY(scratch_t(c, SC_TW, s, &pw));
+      RBT_TRY(scratch_t(c, SC_FLAGS, 4, &nr));
+      const rbt::X3Pick pick{ids, w, (int)s, (int)k, (int)slot->eid, ptok, pw, nr};
+      HIP_OK(c, rbt::launch_x3split(*c, kind, x, s, d, xb3, nullptr, &pick));
+      rbt::X3Args A;
+      A.single = v;
+      A.nrows_dev = nr;
+      A.nrows = A.S = (int)s;
+      A.row_tok = ptok;
+      A.xb3 = xb3;
+      A.tch = s > 48 ? 32 : 16;
+      A.wgs = rbt::x3_wgs(*c, A.tch);
+      A.K = (int)d;
+      A.O = (int)i;
+      A.part = 1;
+      A.hb3 = hb3;
+      A.y = xp;
+      A.act = act;
+      HIP_OK(c, rbt::launch_x3(*c, kind, true, A));
+      HIP_OK(c, rbt::launch_x3act(*c, kind, A));
+      A.row_tok = nullptr;
+      A.xb3 = hb3;
+      A.K = (int)i;
+      A.O = (int)d;
+      HIP_OK(c, rbt::launch_x3(*c, kind, false, A));
+      HIP_OK(c, rbt::launch_x3acc(*c, A, ptok, pw, out));
+      return RBT_OK;
+    }
   }
   int *ptok, *nr;
   float *pw, *h, *yy;

@@ -4,23 +4,10 @@
 
 namespace rbt {
 
-// rows = tokens that picked `eid`, in token order, with their weights (glm52/moe.rs:465-470: the
-// first slot of each token that matches).
-__global__ void k_single_rows(const int32_t *__restrict__ ids, const float *__restrict__ w, int S, int k, int eid,
-                              int *__restrict__ pair_tok, float *__restrict__ pair_w, int *__restrict__ nr) {
-  if (threadIdx.x != 0 || blockIdx.x != 0) return;
-  int n = 0;
-  for (int t = 0; t < S; t++) {
-    for (int j = 0; j < k; j++) {
-      if (ids[t * k + j] == eid) {
-        pair_tok[n] = t;
-        pair_w[n] = w[t * k + j];
-        n++;
-        break;
-      }
-    }
-  }
-  *nr = n;
+__global__ __launch_bounds__(256) void k_single_rows(const int32_t *__restrict__ ids, const float *__restrict__ w, int S,
+                                                     int k, int eid, int *__restrict__ pair_tok,
+                                                     float *__restrict__ pair_w, int *__restrict__ nr) {
+  rbt_single_rows(ids, w, S, k, eid, pair_tok, pair_w, nr);
 }
 
 // out[tok(r), d] += w_r * y[r, d] with separate roundings (glm52/moe.rs:508-512). A token
@@ -37,7 +24,7 @@ __global__ void k_accumulate(const float *__restrict__ y, int S, int H, const in
 
 hipError_t launch_single_rows(const Ctx &c, const int32_t *ids, const float *w, int S, int k, int eid, int *pair_tok,
                               float *pair_w, int *nr) {
-  launch_k(c, k_single_rows, dim3(1), dim3(64), ids, w, S, k, eid, pair_tok, pair_w, nr);
+  launch_k(c, k_single_rows, dim3(1), dim3(256), ids, w, S, k, eid, pair_tok, pair_w, nr);
   return hipGetLastError();
 }
 

@@ -177,6 +177,35 @@ __device__ __forceinline__ double rbt_wave_total_d(double v) {
   return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
 }
 
+// The tokens that picked `eid`, in token order, with their weights (glm52/moe.rs:465-470: the first
+// slot of each token that matches), by one workgroup of 256 threads.
+__device__ __forceinline__ void rbt_single_rows(const int32_t *__restrict__ ids, const float *__restrict__ w, int S,
+                                                int k, int eid, int *__restrict__ pair_tok,
+                                                float *__restrict__ pair_w, int *__restrict__ nr) {
+  __shared__ int cnt[4];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  int base = 0;
+  for (int t0 = 0; t0 < S; t0 += 256) {
+    const int t = t0 + threadIdx.x;
+    int slot = -1;
+    if (t < S)
+      for (int j = k - 1; j >= 0; j--)
+        if (ids[(long)t * k + j] == eid) slot = j;
+    const unsigned long long m = __ballot(slot >= 0);
+    if (lane == 0) cnt[wave] = __popcll(m);
+    __syncthreads();
+    int at = base + __popcll(m & (lane == 0 ? 0ull : ~0ull >> (64 - lane)));
+    for (int i = 0; i < wave; i++) at += cnt[i];
+    if (slot >= 0) {
+      pair_tok[at] = t;
+      pair_w[at] = w[(long)t * k + slot];
+    }
+    base += cnt[0] + cnt[1] + cnt[2] + cnt[3];
+    __syncthreads();
+  }
+  if (threadIdx.x == 0) *nr = base;
+}
+
 // Device view of one expert: gate/up/down as separate (data, scale) pointers. A fused gate_up
 // tensor is presented as two views into the same allocation.
 struct RbtExpertDev {

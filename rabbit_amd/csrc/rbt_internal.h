@@ -218,8 +218,10 @@ struct X3Args {
   const __bf16 *xb3 = nullptr;  // [3 rows, K] parts
   int tch = 16;                 // rows per tile
   int K = 0, O = 0;             // columns, rows of one matrix
-  int KS = 1;                   // K parts (single only): y takes [KS][matrices][nrows, O] partial sums
-  __bf16 *hb3 = nullptr;        // gate/up, KS = 1: act(g, u) as the down product's parts [3 pairs, O]
+  // single only: write partial sums of x3_ks() K parts, y [parts][matrices][rows, O] over the rows there are
+  int part = 0;
+  int wgs = 0;                  // x3_wgs(ctx, tch)
+  __bf16 *hb3 = nullptr;        // gate/up: act(g, u) as the down product's parts [3 pairs, O]
   float *y = nullptr;           // down / matrix: [pairs, O]
   RbtAct act{};
   unsigned *queue = nullptr;  // grouped: 8 cleared counters, units are taken in turn
@@ -229,16 +231,38 @@ constexpr int X3_QN = 16;
 bool x3_ok(int kind, size_t gs, size_t cols, size_t rows, bool gateup);
 // Tiles of launch_pgroup over S tokens, at most.
 long x3_max_tiles(int S, int k, int E, int has_shared, int tch);
-// K parts that fill the chip for n rows through one matrix (or one expert's gate and up).
-int x3_parts(const Ctx &c, size_t n, int tch, size_t cols, size_t rows, bool gateup);
+int x3_wgs(const Ctx &c, int tch);
+// Row blocks of a product: 64 rows of gate and of up, or 128 rows.
+__host__ __device__ inline int x3_row_blocks(int o, bool gateup) { return o / (gateup ? 64 : 128); }
+// K parts (of whole 512 columns) that fill wgs workgroups for n rows, at most X3_KSMAX.
+constexpr int X3_KSMAX = 8;
+__host__ __device__ inline int x3_ks(long n, int tch, int cols, int row_blocks, int wgs) {
+  const long units = (n + tch - 1) / tch * row_blocks, ks = units > 0 ? (wgs + units - 1) / units : 1;
+  const int most = cols / 512 < X3_KSMAX ? cols / 512 : X3_KSMAX;
+  return ks < 1 ? 1 : ks > most ? most : (int)ks;
+}
+// Rows of partial sums (each `matrices` x O floats) that x3_ks can ask for, over every n up to the given one.
+inline size_t x3_part_rows(const Ctx &c, size_t n, int row_blocks) {
+  return 64 * (size_t)c.num_cu / row_blocks + n + 256;
+}
+// One expert's tokens, found beside the split (rbt_single_rows).
+struct X3Pick {
+  const int32_t *ids;
+  const float *w;
+  int S, k, eid;
+  int *pair_tok;
+  float *pair_w;
+  int *nr;
+};
 // x and xb3 16-byte aligned, K a multiple of 8. queue: X3_QN counters to clear (8 per product).
 hipError_t launch_x3split(const Ctx &c, int kind, const float *x, size_t S, size_t K, __bf16 *xb3,
-                          unsigned *queue = nullptr);
+                          unsigned *queue = nullptr, const X3Pick *pick = nullptr);
 hipError_t launch_x3(const Ctx &c, int kind, bool gateup, const X3Args &A);
-// After launch_x3 with KS > 1: y[n] = the sum of the KS partial vectors (n a multiple of 4), or (gate/
-// up) A.hb3 from the partial sums in A.y.
+// After launch_x3 with part: y[n] = the sum of the KS partial vectors (n a multiple of 4); or (gate/up)
+// A.hb3 from the partial sums in A.y; or (down) out[tok[r]] += w[r] * row r's sum, separate roundings.
 hipError_t launch_x3sum(const Ctx &c, const float *part, size_t n, int KS, float *y);
 hipError_t launch_x3act(const Ctx &c, int kind, const X3Args &A);
+hipError_t launch_x3acc(const Ctx &c, const X3Args &A, const int *tok, const float *w, float *out);
 
 // router.hip
 hipError_t launch_router_logits(const Ctx &c, const float *x, int S, int H, const float *W, int E, const float *sgate,

@@ -10,7 +10,8 @@
 //                e4m3's subnormals and first binade), v_cvt_scalef32_pk_bf16_fp8 times 2^9; the group's
 //                scale multiplies the group's fp32 sum.
 // Each product is exact and the sums are fp32: partial sums of 32 columns (int4, the group) or 256
-// (MXFP4) in the MFMA accumulator, then added to the row's sum.
+// (MXFP4) in the MFMA accumulator, then added to the row's sum. Error against 64 bits (2048-8192 columns,
+// 2-norm): MXFP4 0.6-0.9e-7 (the decode GEMV 1.2e-7), int4 1.0-1.4e-7 (2.6-2.9e-7).
 //
 // MFMA operands (v_mfma_f32_16x16x32_bf16): A's 16 rows are activation rows, B's 16 columns weight
 // rows, so that a lane's column, and with it a group's scale, is one weight row. MFMA j of a
@@ -119,9 +120,15 @@ __device__ __forceinline__ void x3_write8(const float (&v)[8], __bf16 *__restric
 }
 
 // x [S, K] fp32 -> xb3 [3 S, K] (row 3 t + part); clears the unit queues of the products that follow.
+// With pick, the last workgroup lists one expert's tokens instead.
 template <bool I4>
 __global__ __launch_bounds__(256) void k_x3split(const float *__restrict__ x, long n8, int k8,
-                                                 __bf16 *__restrict__ xb3, unsigned *__restrict__ queue) {
+                                                 __bf16 *__restrict__ xb3, unsigned *__restrict__ queue,
+                                                 const X3Pick pick) {
+  if (pick.ids && blockIdx.x == gridDim.x - 1) {  // (uniform) a workgroup of its own
+    rbt_single_rows(pick.ids, pick.w, pick.S, pick.k, pick.eid, pick.pair_tok, pick.pair_w, pick.nr);
+    return;
+  }
   if (queue && blockIdx.x == 0 && threadIdx.x < X3_QN) queue[threadIdx.x] = 0u;
   const long i = (long)blockIdx.x * 256 + threadIdx.x;
   if (i >= n8) return;
@@ -215,11 +222,13 @@ __device__ __forceinline__ void x3_run(const uint8_t *src, const uint32_t (&so)[
   stage_store(0);
   stage_load(0);
   __syncthreads();
-  xf4 acc[NT][NQ], ch[NT][NQ];
+  // ch: the chained products; cl (MXFP4, three chained parts): those of the two small parts, so that the
+  // full-size sum rounds once per block and not three times
+  xf4 acc[NT][NQ], ch[NT][NQ], cl[NT][NQ];
 #pragma unroll
   for (int t = 0; t < NT; t++)
 #pragma unroll
-    for (int q = 0; q < NQ; q++) acc[t][q] = ch[t][q] = xf4{0.f, 0.f, 0.f, 0.f};
+    for (int q = 0; q < NQ; q++) acc[t][q] = ch[t][q] = cl[t][q] = xf4{0.f, 0.f, 0.f, 0.f};
   int c_rb = 0, c_g = 0;
   for (int it = 0; it < total; it++) {
     // the group's codes -> the wave's LDS area; its scales: int4 from the lanes holding this quarter of
@@ -272,9 +281,14 @@ __device__ __forceinline__ void x3_run(const uint8_t *src, const uint32_t (&so)[
           const xb8 bv = x3_b<I4>(code, I4 ? 0.0f : rbt_e8m0(((d ? cs[t].y : cs[t].x) >> (8 * j)) & 0xffu));
 #pragma unroll
           for (int q = 0; q < NQ; q++) {
-            xf4 dd = I4 ? xf4{0.f, 0.f, 0.f, 0.f} : ch[t][q];
+            xf4 dd = I4 ? xf4{0.f, 0.f, 0.f, 0.f} : NP == 3 ? cl[t][q] : ch[t][q];
 #pragma unroll
-            for (int p = NP - 1; p >= 0; p--) dd = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[NP * q + p], bv, dd, 0, 0, 0);
+            for (int p = NP - 1; p >= (I4 ? 0 : NP == 3); p--)
+              dd = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[NP * q + p], bv, dd, 0, 0, 0);
+            if (!I4 && NP == 3) {
+              cl[t][q] = dd;
+              dd = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[NP * q], bv, ch[t][q], 0, 0, 0);
+            }
             if (I4) {
 #pragma unroll
               for (int i = 0; i < 4; i++) acc[t][q][i] = __builtin_fmaf(s4[t][j], dd[i], acc[t][q][i]);
@@ -302,8 +316,8 @@ __device__ __forceinline__ void x3_run(const uint8_t *src, const uint32_t (&so)[
 #pragma unroll
         for (int q = 0; q < NQ; q++) {
 #pragma unroll
-          for (int i = 0; i < 4; i++) acc[t][q][i] += ch[t][q][i];
-          ch[t][q] = xf4{0.f, 0.f, 0.f, 0.f};
+          for (int i = 0; i < 4; i++) acc[t][q][i] += NP == 3 ? ch[t][q][i] + cl[t][q][i] : ch[t][q][i];
+          ch[t][q] = cl[t][q] = xf4{0.f, 0.f, 0.f, 0.f};
         }
     }
     if (++c_g == ng) {  // row block done (uniform)
@@ -322,7 +336,10 @@ __device__ __forceinline__ void x3_run(const uint8_t *src, const uint32_t (&so)[
 struct X3Tile {
   RbtExpertDev J;
   int pbase, M;
+  int n;  // single: the rows there are
 };
+__device__ __forceinline__ int x3_rows(const X3Args &A) { return A.nrows_dev ? min(A.nrows, *A.nrows_dev) : A.nrows; }
+
 __device__ __forceinline__ X3Tile x3_tile(const X3Args &A, int ti) {
   X3Tile T;
   if (A.tiles) {
@@ -332,11 +349,12 @@ __device__ __forceinline__ X3Tile x3_tile(const X3Args &A, int ti) {
     T.pbase = s.off + t.c0;
     T.M = min(A.tch, s.cnt - t.c0);
     if (T.J.gd == nullptr || T.J.ud == nullptr || T.J.dd == nullptr) T.M = 0;  // reported by k_pgroup
+    T.n = 0;
   } else {
-    const int n = A.nrows_dev ? min(A.nrows, *A.nrows_dev) : A.nrows;
+    T.n = x3_rows(A);
     T.J = A.single;
     T.pbase = ti * A.tch;
-    T.M = min(A.tch, n - T.pbase);
+    T.M = min(A.tch, T.n - T.pbase);
   }
   return T;
 }
@@ -357,11 +375,11 @@ __device__ __forceinline__ void x3_row(int q, int m, int &tok, int &part) {
 }
 
 template <bool I4, bool GATEUP, int MODE>
-__device__ __forceinline__ void x3_unit(const X3Args &A, const X3Tile &T, int ks, int rb0, int per, uint8_t *lds) {
+__device__ __forceinline__ void x3_unit(const X3Args &A, const X3Tile &T, int KS, int ks, int rb0, uint8_t *lds) {
   constexpr int NM = GATEUP ? 2 : 1, TILES = GATEUP ? 1 : 2, NT = NM * TILES, BR = 64 * TILES;
   constexpr int AR = x3_arows(MODE), NQ = MODE == X3_BIG ? 2 : 1;
   const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4, w = threadIdx.x >> 6;
-  const int K = A.K, O = A.O, KS = A.KS, n2 = K / (2 * X3_KG);
+  const int K = A.K, O = A.O, n2 = K / (2 * X3_KG);
   const int g0 = ks * n2 / KS * 2, g1 = (ks + 1) * n2 / KS * 2;  // K parts of whole 512 columns
   // activation rows: a token's through row_tok from the call's first row, else from the tile's first
   const long row0 = A.row_tok ? 0 : T.pbase;
@@ -382,16 +400,16 @@ __device__ __forceinline__ void x3_unit(const X3Args &A, const X3Tile &T, int ks
   } else {
     wa[0] = T.J.dd, ws[0] = (const uint8_t *)T.J.ds;
   }
-  x3_run<I4, NM, TILES, MODE>(src, so, wa, ws, K, rb0, per, g0, g1 - g0, lds, [&](int rb, xf4(&acc)[NT][NQ]) {
+  x3_run<I4, NM, TILES, MODE>(src, so, wa, ws, K, rb0, 1, g0, g1 - g0, lds, [&](int rb, xf4(&acc)[NT][NQ]) {
     const int o0 = rb * BR + 16 * TILES * w + r;
     // v[t]: token tok's sum of weight tile t, row o0 + 16 (t % TILES)
     auto put = [&](int tok, const float(&v)[NT]) {
       if (tok >= T.M) return;
       const long pr = T.pbase + tok;
-      if (KS > 1) {
+      if (A.part) {
 #pragma unroll
         for (int t = 0; t < NT; t++)
-          A.y[((long)(ks * NM + t / TILES) * A.nrows + pr) * O + o0 + 16 * (t % TILES)] = v[t];
+          A.y[((long)(ks * NM + t / TILES) * T.n + pr) * O + o0 + 16 * (t % TILES)] = v[t];
       } else if (GATEUP) {
         __bf16 p[3];
         x3_split(rbt_act(A.act, v[0], v[NT - 1]), p);
@@ -437,8 +455,9 @@ __device__ __forceinline__ void x3_unit(const X3Args &A, const X3Tile &T, int ks
 template <bool I4, bool GATEUP, int TOP>
 __global__ __launch_bounds__(256, TOP == X3_BIG ? 2 : 3) void k_x3(const X3Args A) {
   __shared__ __attribute__((aligned(16))) uint8_t lds[x3_lds_bytes(I4, TOP)];
-  const int RB = A.O / (GATEUP ? 64 : 128), KS = A.KS;
-  const int nt = A.tiles ? *A.ntiles : (A.nrows + A.tch - 1) / A.tch;
+  const int RB = x3_row_blocks(A.O, GATEUP), rows = A.tiles ? 0 : x3_rows(A);
+  const int KS = A.part ? x3_ks(rows, A.tch, A.K, RB, A.wgs) : 1;
+  const int nt = A.tiles ? *A.ntiles : (rows + A.tch - 1) / A.tch;
   const long U = (long)nt * RB * KS;
   const int xcd = blockIdx.x & 7, nx = gridDim.x >> 3;
   __shared__ int next_s;
@@ -453,11 +472,11 @@ __global__ __launch_bounds__(256, TOP == X3_BIG ? 2 : 3) void k_x3(const X3Args 
     const X3Tile T = x3_tile(A, ti);
     if (T.M <= 0) {
     } else if (T.M <= 5)
-      x3_unit<I4, GATEUP, X3_SMALL>(A, T, ks, rb0, 1, lds);
+      x3_unit<I4, GATEUP, X3_SMALL>(A, T, KS, ks, rb0, lds);
     else if (TOP == X3_MID || T.M <= 16)
-      x3_unit<I4, GATEUP, X3_MID>(A, T, ks, rb0, 1, lds);
+      x3_unit<I4, GATEUP, X3_MID>(A, T, KS, ks, rb0, lds);
     else
-      x3_unit<I4, GATEUP, X3_BIG>(A, T, ks, rb0, 1, lds);
+      x3_unit<I4, GATEUP, X3_BIG>(A, T, KS, ks, rb0, lds);
     if (A.queue) {
       __syncthreads();
       if (threadIdx.x == 0) next_s = nx + (int)taken;
@@ -482,30 +501,60 @@ __global__ __launch_bounds__(256) void k_x3sum(const xf4 *__restrict__ part, lon
   y[i] = v;
 }
 
-// Gate/up: h = act(sum of gate parts, sum of up parts), as the down product's activation parts.
-// One thread per 8 columns of a row; rows past *nrows_dev are left alone.
+// Gate/up: h = act(sum of gate parts, sum of up parts), as the down product's activation parts. Four
+// threads per 8 columns of a row, each summing every fourth part (one thread summing them all waits for
+// memory once per part: 12.6 us at 16 parts); rows past *nrows_dev are left alone.
 template <bool I4>
 __global__ __launch_bounds__(256) void k_x3act(const X3Args A) {
-  const int o8 = A.O >> 3;
-  const long i = (long)blockIdx.x * 256 + threadIdx.x;
-  const int n = A.nrows_dev ? min(A.nrows, *A.nrows_dev) : A.nrows;
+  const int o8 = A.O >> 3, q4 = threadIdx.x & 3;
+  const long i = ((long)blockIdx.x * 256 + threadIdx.x) >> 2;
+  const int n = x3_rows(A), KS = x3_ks(n, A.tch, A.K, x3_row_blocks(A.O, true), A.wgs);
   const long pr = i / o8;
-  if (pr >= n) return;
+  if (pr >= n) return;  // the four threads together
   const long c = 8 * (i - pr * o8);
   float gu[2][8] = {};
-  for (int p = 0; p < A.KS; p++)
+  for (int p = q4; p < KS; p += 4)
 #pragma unroll
     for (int m = 0; m < 2; m++)
 #pragma unroll
       for (int q = 0; q < 2; q++) {
-        const xf4 v = *reinterpret_cast<const xf4 *>(A.y + ((long)(p * 2 + m) * A.nrows + pr) * A.O + c + 4 * q);
+        const xf4 v = *reinterpret_cast<const xf4 *>(A.y + ((long)(p * 2 + m) * n + pr) * A.O + c + 4 * q);
 #pragma unroll
         for (int e = 0; e < 4; e++) gu[m][4 * q + e] += v[e];
       }
+#pragma unroll
+  for (int m = 0; m < 2; m++)
+#pragma unroll
+    for (int e = 0; e < 8; e++) {
+      gu[m][e] = rbt_dpp_add<0xB1>(gu[m][e]);  // quad_perm: xor 1, xor 2
+      gu[m][e] = rbt_dpp_add<0x4E>(gu[m][e]);
+    }
+  if (q4) return;
   float h[8];
 #pragma unroll
   for (int e = 0; e < 8; e++) h[e] = rbt_act(A.act, gu[0][e], gu[1][e]);
   x3_write8<I4>(h, A.hb3 + 3 * pr * A.O + c, A.O);
+}
+
+// One expert's weighted rows into the tokens' (glm52/moe.rs:508-512); a token appears at most once.
+__global__ __launch_bounds__(256) void k_x3acc(const X3Args A, const int *__restrict__ tok,
+                                               const float *__restrict__ w, float *__restrict__ out) {
+  const int o4 = A.O >> 2;
+  const long i = (long)blockIdx.x * 256 + threadIdx.x;
+  const int n = x3_rows(A), KS = x3_ks(n, A.tch, A.K, x3_row_blocks(A.O, false), A.wgs);
+  const long r = i / o4;
+  if (r >= n) return;
+  const xf4 *part = reinterpret_cast<const xf4 *>(A.y);
+  xf4 v = part[i];
+  for (int p = 1; p < KS; p++) {
+    const xf4 q = part[(long)p * n * o4 + i];
+#pragma unroll
+    for (int e = 0; e < 4; e++) v[e] += q[e];
+  }
+  float *o = out + (long)tok[r] * A.O + 4 * (i - r * o4);
+  const float wr = w[r];
+#pragma unroll
+  for (int e = 0; e < 4; e++) o[e] = __fadd_rn(o[e], __fmul_rn(wr, v[e]));
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -524,27 +573,23 @@ long x3_max_tiles(int S, int k, int E, int has_shared, int tch) {
 }
 
 // workgroups, a multiple of 8
-static int x3_wgs(const Ctx &c, int tch) { return ((tch > 16 ? 2 : 3) * c.num_cu + 7) / 8 * 8; }
+int x3_wgs(const Ctx &c, int tch) { return ((tch > 16 ? 2 : 3) * c.num_cu + 7) / 8 * 8; }
 
-int x3_parts(const Ctx &c, size_t n, int tch, size_t cols, size_t rows, bool gateup) {
-  const long units = (long)((n + tch - 1) / tch) * (long)(rows / (gateup ? 64 : 128));
-  const long ng = (long)cols / (2 * X3_KG);
-  return (int)std::max(1L, std::min(ng, (x3_wgs(c, tch) + units - 1) / units));
-}
-
-hipError_t launch_x3split(const Ctx &c, int kind, const float *x, size_t S, size_t K, __bf16 *xb3, unsigned *queue) {
+hipError_t launch_x3split(const Ctx &c, int kind, const float *x, size_t S, size_t K, __bf16 *xb3, unsigned *queue,
+                          const X3Pick *pick) {
   const long n8 = (long)(S * K / 8);
   if (n8 <= 0) return hipSuccess;
-  const dim3 grid((unsigned)((n8 + 255) / 256));
+  const dim3 grid((unsigned)((n8 + 255) / 256 + (pick ? 1 : 0)));
+  const X3Pick p = pick ? *pick : X3Pick{};
   if (kind == RBT_QT_I4_GROUPED)
-    launch_k(c, k_x3split<true>, grid, dim3(256), x, n8, (int)(K / 8), xb3, queue);
+    launch_k(c, k_x3split<true>, grid, dim3(256), x, n8, (int)(K / 8), xb3, queue, p);
   else
-    launch_k(c, k_x3split<false>, grid, dim3(256), x, n8, (int)(K / 8), xb3, queue);
+    launch_k(c, k_x3split<false>, grid, dim3(256), x, n8, (int)(K / 8), xb3, queue, p);
   return hipGetLastError();
 }
 
 hipError_t launch_x3(const Ctx &c, int kind, bool gateup, const X3Args &A) {
-  if (A.K % (2 * X3_KG) || A.O % (gateup ? 64 : 128) || A.KS < 1) return hipErrorInvalidValue;
+  if (A.K % (2 * X3_KG) || A.O % (gateup ? 64 : 128) ) return hipErrorInvalidValue;
 
   if ((A.tch != 16 && A.tch != 32) || 6L * A.S * A.K >= (1L << 32)) return hipErrorInvalidValue;
   const dim3 grid(x3_wgs(c, A.tch)), blk(256);
@@ -571,8 +616,14 @@ hipError_t launch_x3sum(const Ctx &c, const float *part, size_t n, int KS, float
   return hipGetLastError();
 }
 
+hipError_t launch_x3acc(const Ctx &c, const X3Args &A, const int *tok, const float *w, float *out) {
+  const long n = (long)A.nrows * (A.O / 4);
+  launch_k(c, k_x3acc, dim3((unsigned)((n + 255) / 256)), dim3(256), A, tok, w, out);
+  return hipGetLastError();
+}
+
 hipError_t launch_x3act(const Ctx &c, int kind, const X3Args &A) {
-  const long n = (long)A.nrows * (A.O / 8);
+  const long n = (long)A.nrows * (A.O / 8) * 4;
   const dim3 grid((unsigned)((n + 255) / 256));
   if (kind == RBT_QT_I4_GROUPED)
     launch_k(c, k_x3act<true>, grid, dim3(256), A);

@@ -99,3 +99,32 @@ def test_latent_batches(ctx, orc, E, k, S):
     x = normal((S, H), S, 1.0)
     norm = np.abs(normal(MH, 5, 1.0)) + np.float32(0.5)
     _run_latent(ctx, R, layer, L, dq, uq, x, S, MH, norm, orc.situ(4.0, 25.0), R.situ(4.0, 25.0))
+
+
+# nobody, one, 5, 6, 16, 17, 33 and 300 of the tokens pick the expert; K parts on both products
+@pytest.mark.parametrize("fmt,d,i", [("mxfp4", 8192, 2048), ("i4g", 512, 512)])
+@pytest.mark.parametrize("s,picks", [(9, 0), (5, 1), (7, 5), (20, 6), (16, 16), (47, 17), (49, 33), (300, 300)])
+def test_expert_batches(ctx, orc, fmt, d, i, s, picks):
+    import torch
+    import rabbit_amd as R
+    (g, gd), (u, ud), (dn, dd) = (_matrix(ctx, orc, fmt, r, c, 11 + r + n) for n, (r, c) in
+                                  enumerate(((i, d), (i, d), (d, i))))
+    rng = np.random.default_rng(s)
+    k = 3
+    ids = rng.integers(1, 50, (s, k)).astype(np.int32)
+    who = np.sort(rng.permutation(s)[:picks])
+    ids[who, rng.integers(0, k, picks)] = 0
+    ids[who[::2], k - 1] = 0  # some pick it twice: the first slot counts
+    w = rng.standard_normal((s, k)).astype(np.float32)
+    x = torch.from_numpy(normal((s, d), s)).cuda()
+    out = torch.full((s, d), 0.5, device="cuda")
+    slot = R.Slot(0, dn, gate=g, up=u)
+    ctx.apply_single_expert(slot, torch.from_numpy(ids).cuda(), torch.from_numpy(w).cuda(), s, k, x, d, i, out)
+    want = torch.full((s, d), 0.5, dtype=torch.float64, device="cuda")
+    for t in who:
+        h = torch.nn.functional.silu(gd @ x[t].double()) * (ud @ x[t].double())
+        want[t] += float(w[t, list(ids[t]).index(0)]) * (dd @ h)
+    assert float((out.double() - want).norm() / want.norm()) < 1e-6
+    rest = torch.ones(s, dtype=torch.bool)
+    rest[torch.from_numpy(who)] = False
+    assert bool((out[rest.cuda()] == 0.5).all())
