@@ -292,7 +292,13 @@ __device__ __forceinline__ void pf_decode(const PfA &a, int g, pb8 (&A)[4]) {
 }
 
 constexpr int PF_RBG = 8;         // workgroups per tile: each takes 1/8 of the rows (contiguous)
-constexpr int PB_STRIDE = 128 + 8;  // bf16 per LDS token row of a step (272 B: rows 4 banks apart)
+// LDS layout of the wider prefill tiles (17 tokens and more): activation rows 288 B apart, and a weight
+// row's 16-byte piece p at p ^ row, so that reading 16 rows covers all banks (35% fewer conflict cycles).
+// Those tiles are bound by LDS and the matrix cores: 1537 tokens gate/up 2479 -> 2170-2300 us, down 1472 ->
+// 1310-1350, with a form of their own for tiles of 33-48 tokens. Tiles of up to 16 tokens and the grouped
+// decode are bound by the weight stream, where the index arithmetic costs 1-2%: rows 272 B apart.
+constexpr bool pf_swz(bool dec, int ntv) { return !dec && ntv > 1; }
+constexpr int pb_stride(bool dec, int ntv) { return 128 + (pf_swz(dec, ntv) ? 16 : 8); }  // bf16 per token row of a step
 
 // The tile's activations for one K step (nt * 16 tokens x 128 columns, bf16) go through LDS: the
 // workgroup loads them with one coalesced 16-byte load per thread per 16 tokens (a token's 256
@@ -315,15 +321,16 @@ __device__ __forceinline__ void pf_stage_load(PfStage<NTV> &st, const __bf16 *co
   for (int q = 0; q < NTV; q++) st.v[q] = *(const rbt_gu4 *)(src[q] + 128 * s);
 }
 
-template <int NTV>
-__device__ __forceinline__ void pf_stage_store(const PfStage<NTV> &st, __bf16 (*buf)[PB_STRIDE]) {
+template <int NTV, int PB>
+__device__ __forceinline__ void pf_stage_store(const PfStage<NTV> &st, __bf16 (*buf)[PB]) {
   const int j = threadIdx.x >> 4, c = (threadIdx.x & 15) * 8;
 #pragma unroll
   for (int q = 0; q < NTV; q++) *reinterpret_cast<rbt_u4 *>(&buf[16 * q + j][c]) = st.v[q];
 }
 
 // B operand of MFMA m for column block q: token 16 q + r, columns 32 g + 8 m .. +7 of the step.
-__device__ __forceinline__ pb8 pf_b(const __bf16 (*buf)[PB_STRIDE], int q, int m, int r, int g) {
+template <int PB>
+__device__ __forceinline__ pb8 pf_b(const __bf16 (*buf)[PB], int q, int m, int r, int g) {
   return *reinterpret_cast<const pb8 *>(&buf[16 * q + r][32 * g + 8 * m]);
 }
 
@@ -331,17 +338,17 @@ __device__ __forceinline__ pb8 pf_b(const __bf16 (*buf)[PB_STRIDE], int q, int m
 // at about two thirds of the bandwidth of 4 rows x 256 contiguous bytes on this part. So each
 // wave loads its tiles' K groups (4 steps = 256 bytes per row) as 4 rows x 256 bytes per
 // instruction (lane l: row 4 q + l / 16 of the 16-row tile, bytes 16 (l % 16) .. +15 of the group),
-// writes them to its own LDS area at a PW_STRIDE-byte row stride, and every step reads the MFMA
+// writes them to its own LDS area at a pw_stride-byte row stride, and every step reads the MFMA
 // layout back (lane (r, g): row r, bytes 16 (4 d + g) .. +15 of step d). The 272-byte stride puts
 // the 16 rows of a read 4 banks apart, and a wave reads its area only after its own writes, in
 // order, so no barrier is needed.
-constexpr int PW_STRIDE = 256 + 16;       // bytes per staged weight row (one K group)
-constexpr int PW_TILE = 16 * PW_STRIDE;   // bytes per staged 16-row tile
+constexpr int pw_stride(bool dec, int ntv) { return 256 + (pf_swz(dec, ntv) ? 0 : 16); }  // bytes per staged weight row
+constexpr int pw_tile(bool dec, int ntv) { return 16 * pw_stride(dec, ntv); }  // bytes per staged 16-row tile
 
 // LDS of one pf_gemm workgroup: the activation double buffer (2 x 16 NTV token rows) then each
 // wave's staged weights (NM TILES tiles).
-constexpr int pf_lds_bytes(int NM, int NTV, int TILES) {
-  return 2 * 16 * NTV * PB_STRIDE * 2 + 4 * NM * TILES * PW_TILE;
+constexpr int pf_lds_bytes(int NM, int NTV, int TILES, bool dec = false) {
+  return 2 * 16 * NTV * pb_stride(dec, NTV) * 2 + 4 * NM * TILES * pw_tile(dec, NTV);
 }
 
 // One tile x row-block group. Wave w owns TILES 16-row tiles (16 TILES contiguous rows) of each
@@ -367,6 +374,8 @@ __device__ __forceinline__ void pf_gemm(const PfTile &T, const __bf16 *const (&s
                                         int nsteps, int out_cols, __bf16 *__restrict__ hb, float *__restrict__ y,
                                         uint8_t *lds, int rbs = PF_RBG) {
   constexpr int G = 4;  // K steps per group
+  constexpr int PB_STRIDE = pb_stride(DEC, NTV), PW_STRIDE = pw_stride(DEC, NTV), PW_TILE = pw_tile(DEC, NTV);
+  constexpr bool SWZ = pf_swz(DEC, NTV);
   const int w = threadIdx.x >> 6, lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
   constexpr int BR = 64 * TILES;                                         // rows per row block
   const long blk_a = (long)rbs * BR * rowb, blk_s = (long)rbs * BR * rows;  // between own blocks
@@ -441,7 +450,7 @@ __device__ __forceinline__ void pf_gemm(const PfTile &T, const __bf16 *const (&s
     for (int d = 0; d < G; d++) stage_next(st[(d + 1) % G]);
     if (sline) sl_load(0, 0);
     fetch_group();
-    pf_stage_store<NTV>(s0, bs[0]);
+    pf_stage_store<NTV, PB_STRIDE>(s0, bs[0]);
   }
   __syncthreads();
   pf4 acc[NM][TILES][NTV];
@@ -478,28 +487,29 @@ __device__ __forceinline__ void pf_gemm(const PfTile &T, const __bf16 *const (&s
 #pragma unroll
       for (int t = 0; t < TILES; t++) {
         if (!sline) cs[m][t] = ns[m][t];
-        uint8_t *wt = wl + (m * TILES + t) * PW_TILE + (lane >> 4) * PW_STRIDE + 16 * (lane & 15);
+        uint8_t *wt = wl + (m * TILES + t) * PW_TILE + (lane >> 4) * PW_STRIDE;
 #pragma unroll
-        for (int q = 0; q < 4; q++) *reinterpret_cast<rbt_u4 *>(wt + 4 * q * PW_STRIDE) = nw[m][t][q];
+        for (int q = 0; q < 4; q++)
+          *reinterpret_cast<rbt_u4 *>(wt + 4 * q * PW_STRIDE + 16 * ((lane & 15) ^ (SWZ ? 4 * q + (lane >> 4) : 0))) = nw[m][t][q];
       }
     fetch_group();
 #pragma unroll
     for (int d = 0; d < G; d++) {
       const int buf = d & 1;  // iteration it reads LDS buffer it & 1 (nsteps even)
       // activations of it + 1 (loaded a group ago) -> the other LDS buffer
-      pf_stage_store<NTV>(st[(d + 1) % G], bs[buf ^ 1]);
+      pf_stage_store<NTV, PB_STRIDE>(st[(d + 1) % G], bs[buf ^ 1]);
       stage_next(st[(d + 1) % G]);
       rbt_u4 cw[NM][TILES];
 #pragma unroll
       for (int m = 0; m < NM; m++)
 #pragma unroll
         for (int t = 0; t < TILES; t++)
-          cw[m][t] = *reinterpret_cast<const rbt_u4 *>(wl + (m * TILES + t) * PW_TILE + r * PW_STRIDE + 16 * (4 * d + g));
+          cw[m][t] = *reinterpret_cast<const rbt_u4 *>(wl + (m * TILES + t) * PW_TILE + r * PW_STRIDE + 16 * ((4 * d + g) ^ (SWZ ? r : 0)));
 #pragma unroll
       for (int k4 = 0; k4 < 4; k4++) {
         pb8 bv[NTV];
 #pragma unroll
-        for (int q = 0; q < NTV; q++) bv[q] = pf_b(bs[buf], q, k4, r, g);
+        for (int q = 0; q < NTV; q++) bv[q] = pf_b<PB_STRIDE>(bs[buf], q, k4, r, g);
 #pragma unroll
         for (int m = 0; m < NM; m++)
 #pragma unroll
@@ -660,6 +670,10 @@ __global__ __launch_bounds__(256) void k_pgateup(const PTile *__restrict__ tiles
       const __bf16 *src[2] = {src_of(0), src_of(1)};
       pf_gemm<2, 2, 1>(T, src, a, sc, rowb, rows, gi, per_of(64), nsteps, I, hb, nullptr, lds);
     } break;
+    case 3: {
+      const __bf16 *src[3] = {src_of(0), src_of(1), src_of(2)};
+      pf_gemm<2, 3, 1>(T, src, a, sc, rowb, rows, gi, per_of(64), nsteps, I, hb, nullptr, lds);
+    } break;
     default: {
       const __bf16 *src[4] = {src_of(0), src_of(1), src_of(2), src_of(3)};
       pf_gemm<2, 4, 1>(T, src, a, sc, rowb, rows, gi, per_of(64), nsteps, I, hb, nullptr, lds);
@@ -696,6 +710,10 @@ __global__ __launch_bounds__(256) void k_pdown(const PTile *__restrict__ tiles, 
     case 2: {
       const __bf16 *src[2] = {src_of(0), src_of(1)};
       pf_gemm<1, 2, 2, false, true>(T, src, a, sc, rowb, rows, gi, per_of(128), nsteps, H, nullptr, y, lds, PF_DN_RBG);
+    } break;
+    case 3: {
+      const __bf16 *src[3] = {src_of(0), src_of(1), src_of(2)};
+      pf_gemm<1, 3, 1, false, true>(T, src, a, sc, rowb, rows, gi, per_of(64), nsteps, H, nullptr, y, lds, PF_DN_RBG);
     } break;
     default: {
       const __bf16 *src[4] = {src_of(0), src_of(1), src_of(2), src_of(3)};
@@ -799,7 +817,7 @@ __global__ __launch_bounds__(256) void k_dgateup(const PTile *__restrict__ tiles
                                                  const RbtExpertDev *__restrict__ shared_dev,
                                                  const int *__restrict__ pair_tok, const __bf16 *__restrict__ xb3,
                                                  int S, int H, int I, __bf16 *__restrict__ hb3) {
-  __shared__ __attribute__((aligned(16))) uint8_t lds[pf_lds_bytes(2, 2, 1)];
+  __shared__ __attribute__((aligned(16))) uint8_t lds[pf_lds_bytes(2, 2, 1, true)];
   pd_units<true>(tiles, ntiles, segs, table, shared_dev, pair_tok, xb3, S, H, I, I / 64, hb3, nullptr, lds);
 }
 
@@ -808,7 +826,7 @@ __global__ __launch_bounds__(256) void k_ddown(const PTile *__restrict__ tiles, 
                                                const PSeg *__restrict__ segs, const RbtExpertDev *__restrict__ table,
                                                const RbtExpertDev *__restrict__ shared_dev,
                                                const __bf16 *__restrict__ hb3, int I, int H, float *__restrict__ y) {
-  __shared__ __attribute__((aligned(16))) uint8_t lds[pf_lds_bytes(1, 2, 2)];
+  __shared__ __attribute__((aligned(16))) uint8_t lds[pf_lds_bytes(1, 2, 2, true)];
   pd_units<false>(tiles, ntiles, segs, table, shared_dev, nullptr, hb3, 0, I, H, H / 128, nullptr, y, lds);
 }
 
