@@ -76,6 +76,36 @@ __device__ __forceinline__ uint32_t pg_load(const uint32_t *p) {
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
+// Pair of pick p = t k + j. The slot of (t, e) within e's segment is the number of earlier tokens that
+// picked e. Token t's picks are written in pair order, which is unique_experts order (segments are in
+// rank order): pick j goes to position #{j' : key(j') < key(j)}, with key = rank of the expert, and
+// missing picks after every real one in slot order.
+template <typename RANK, typename OFF>
+__device__ __forceinline__ void pg_pair(int p, const int32_t *__restrict__ ids, const float *__restrict__ wts, int k,
+                                        int E, int W, int P, int has_shared, RANK rank, OFF off, const uint32_t *bits,
+                                        const uint32_t *pc, int *__restrict__ pair_tok, int *__restrict__ tok_pair,
+                                        float *__restrict__ tok_w) {
+  const int t = p / k, j = p - t * k;
+  const int32_t *ti = ids + (long)t * k;
+  const int e = ti[j];
+  const bool v = e >= 0 && e < E;
+  const int kj = v ? rank(e) : E + j;
+  int pos = 0;
+  for (int j2 = 0; j2 < k; j2++) {
+    const int e2 = ti[j2];
+    pos += ((e2 >= 0 && e2 < E) ? rank(e2) : E + j2) < kj;
+  }
+  int pr = -1;
+  if (v) {
+    const long wi = (long)e * W + (t >> 5);
+    pr = off(e) + (int)(pc[wi] + __popc(bits[wi] & ((1u << (t & 31)) - 1u)));
+    pair_tok[pr] = t;
+  }
+  tok_pair[(long)t * k + pos] = pr;
+  tok_w[(long)t * k + pos] = v ? wts[(long)t * k + j] : 0.0f;
+  if (has_shared && j == 0) pair_tok[P + t] = t;
+}
+
 // One workgroup of 1024 threads. ids / wts are [S, k] (id -1 = no pick). bits / pc are scratch of
 // E * ceil(S/32) words each. Outputs:
 //   segs[u]     u < U: unique expert u (first-occurrence order), its pair offset and token count;
@@ -86,7 +116,7 @@ __device__ __forceinline__ uint32_t pg_load(const uint32_t *p) {
 //   tok_pair / tok_w [t*k + j]: token t's pairs and routing weights sorted by pair index, i.e. in
 //               unique_experts order (-1 / 0 for missing picks, placed last).
 // SMALL (E * ceil(S / 32) <= PG_SMALLW): the token bitmaps and their prefix counts live in LDS
-// (bits / pc unused); otherwise in the global scratch.
+// (bits / pc unused); otherwise in the global scratch, and k_ppairs writes the pairs.
 constexpr int PG_SMALLW = 8192;  // words: C4 (512 experts x 512 tokens) keeps its bitmaps in LDS
 template <bool SMALL>
 __global__ __launch_bounds__(1024) void k_pgroup(const int32_t *__restrict__ ids, const float *__restrict__ wts, int S,
@@ -170,12 +200,16 @@ __global__ __launch_bounds__(1024) void k_pgroup(const int32_t *__restrict__ ids
     int tot;
     const int ex = pg_block_scan(n0 + n1, ws, &tot);
     if (u0 < nseg) {
-      segs[u0] = PSeg{u0 < U ? byrank[u0] : -1, u0 < U ? segoff[u0] : P, seg_cnt(u0), 0};
+      segs[u0] = PSeg{u0 < U ? byrank[u0] : -1, u0 < U ? segoff[u0] : P, seg_cnt(u0), !SMALL && u0 < E ? rank[u0] : 0};
       for (int c = 0; c < n0; c++) tiles[ex + c] = PTile{u0, c * tch};
+    } else if (!SMALL && u0 < E) {
+      segs[u0].rank = rank[u0];
     }
     if (u1 < nseg) {
-      segs[u1] = PSeg{u1 < U ? byrank[u1] : -1, u1 < U ? segoff[u1] : P, seg_cnt(u1), 0};
+      segs[u1] = PSeg{u1 < U ? byrank[u1] : -1, u1 < U ? segoff[u1] : P, seg_cnt(u1), !SMALL && u1 < E ? rank[u1] : 0};
       for (int c = 0; c < n1; c++) tiles[ex + n0 + c] = PTile{u1, c * tch};
+    } else if (!SMALL && u1 < E) {
+      segs[u1].rank = rank[u1];
     }
     if (tid == 0) {
       *ntiles = tot;
@@ -186,40 +220,36 @@ __global__ __launch_bounds__(1024) void k_pgroup(const int32_t *__restrict__ ids
   for (int e = tid; e < E; e += 1024) {
     if (cnt[e] == 0) continue;
     uint32_t run = 0;
-    for (int w = 0; w < W; w++) {
-      pc[(long)e * W + w] = run;
-      run += __popc(bload(&bits[(long)e * W + w]));
+    constexpr int NW = SMALL ? 1 : 8;  // global words: eight loads at a time
+    for (int w0 = 0; w0 < W; w0 += NW) {
+      uint32_t v[NW];
+#pragma unroll
+      for (int j = 0; j < NW; j++) v[j] = w0 + j < W ? bload(&bits[(long)e * W + w0 + j]) : 0u;
+#pragma unroll
+      for (int j = 0; j < NW; j++) {
+        if (w0 + j < W) pc[(long)e * W + w0 + j] = run;
+        run += __popc(v[j]);
+      }
     }
   }
-  if (!SMALL) __threadfence();
+  if (!SMALL) return;  // k_ppairs places the pairs
   __syncthreads();
-  // Pairs, one thread per (token, pick). The slot of (t, e) within e's segment is the number of
-  // earlier tokens that picked e. Token t's picks are written in pair order, which is
-  // unique_experts order (segments are in rank order): pick j goes to position
-  // #{j' : key(j') < key(j)}, with key = rank of the expert, and missing picks after every real one
-  // in slot order.
-  for (int p = tid; p < P; p += 1024) {
-    const int t = p / k, j = p - t * k;
-    const int32_t *ti = ids + (long)t * k;
-    const int e = ti[j];
-    const bool v = e >= 0 && e < E;
-    const int kj = v ? rank[e] : E + j;
-    int pos = 0;
-    for (int j2 = 0; j2 < k; j2++) {
-      const int e2 = ti[j2];
-      pos += ((e2 >= 0 && e2 < E) ? rank[e2] : E + j2) < kj;
-    }
-    int pr = -1;
-    if (v) {
-      const long wi = (long)e * W + (t >> 5);
-      const int slot = (int)(bload(&pc[wi]) + __popc(bload(&bits[wi]) & ((1u << (t & 31)) - 1u)));
-      pr = segoff[rank[e]] + slot;
-      pair_tok[pr] = t;
-    }
-    tok_pair[(long)t * k + pos] = pr;
-    tok_w[(long)t * k + pos] = v ? wts[(long)t * k + j] : 0.0f;
-    if (has_shared && j == 0) pair_tok[P + t] = t;
-  }
+  for (int p = tid; p < P; p += 1024)
+    pg_pair(p, ids, wts, k, E, W, P, has_shared, [&](int e) { return rank[e]; }, [&](int e) { return segoff[rank[e]]; },
+            bits, pc, pair_tok, tok_pair, tok_w);
+}
+
+// The pairs of a call whose bitmaps are in global memory, one thread per (token, pick) over the chip: on
+// k_pgroup's one workgroup they took about 50 of its 172 us at 1537 tokens x 10.
+__global__ __launch_bounds__(256) void k_ppairs(const int32_t *__restrict__ ids, const float *__restrict__ wts, int S,
+                                                int k, int E, int has_shared, const PSeg *__restrict__ segs,
+                                                const uint32_t *__restrict__ bits, const uint32_t *__restrict__ pc,
+                                                int *__restrict__ pair_tok, int *__restrict__ tok_pair,
+                                                float *__restrict__ tok_w) {
+  const int p = blockIdx.x * 256 + threadIdx.x;
+  if (p >= S * k) return;
+  pg_pair(p, ids, wts, k, E, (S + 31) >> 5, S * k, has_shared, [&](int e) { return segs[e].rank; },
+          [&](int e) { return segs[segs[e].rank].off; }, bits, pc, pair_tok, tok_pair, tok_w);
 }
 
 // x (fp32) -> bf16, round to nearest even. vec: x and xb allow 16- and 8-byte accesses.
@@ -851,12 +881,15 @@ hipError_t launch_pgroup(const Ctx &c, const int32_t *ids, const float *wts, int
                          const RbtExpertDev *table, uint32_t *bits, uint32_t *pc, PSeg *segs, PTile *tiles,
                          int *ntiles, int *pair_tok, int *tok_pair, float *tok_w, int *err, int *nuniq, int tch) {
   if (E > PG_MAXE || tch < 1) return hipErrorInvalidValue;
-  if ((long)E * ((S + 31) / 32) <= PG_SMALLW)
+  if ((long)E * ((S + 31) / 32) <= PG_SMALLW) {
     launch_k(c, k_pgroup<true>, dim3(1), dim3(1024), ids, wts, S, k, E, has_shared, table, bits, pc, segs, tiles,
              ntiles, pair_tok, tok_pair, tok_w, err, nuniq, tch);
-  else
+  } else {
     launch_k(c, k_pgroup<false>, dim3(1), dim3(1024), ids, wts, S, k, E, has_shared, table, bits, pc, segs, tiles,
              ntiles, pair_tok, tok_pair, tok_w, err, nuniq, tch);
+    launch_k(c, k_ppairs, dim3((unsigned)(((long)S * k + 255) / 256)), dim3(256), ids, wts, S, k, E, has_shared,
+             (const PSeg *)segs, (const uint32_t *)bits, (const uint32_t *)pc, pair_tok, tok_pair, tok_w);
+  }
   return hipGetLastError();
 }
 

@@ -128,3 +128,17 @@ def test_expert_batches(ctx, orc, fmt, d, i, s, picks):
     rest = torch.ones(s, dtype=torch.bool)
     rest[torch.from_numpy(who)] = False
     assert bool((out[rest.cuda()] == 0.5).all())
+
+
+def test_grouping_past_the_lds_bitmaps(ctx, orc):
+    """More (expert, 32-token word) bitmap words than one workgroup's LDS holds: the pairs come from their own
+    launch. Unused experts on both ends of the ids, and a shared expert."""
+    import rabbit_amd as R
+    H, I, E, k, S = 512, 1024, 500, 3, 545
+    L = _small_layer(ctx, orc, 0, R.QT_MXFP4, H, I, E, k, seed=77, gated=True)
+    x = normal((S, H), 9)
+    exp, eids, _ = L.forward(x, S)
+    out, ids, w = np.empty(S * H, np.float32), np.empty(S * k, np.int32), np.empty(S * k, np.float32)
+    ctx.moe_forward(0, x, S, out, ids, w)
+    assert np.array_equal(ids.reshape(S, k), eids)
+    assert rel_l2(out, exp) < 1e-2  # bf16 activations
