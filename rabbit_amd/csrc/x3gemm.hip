@@ -142,26 +142,23 @@ __global__ __launch_bounds__(256) void k_x3split(const float *__restrict__ x, lo
   x3_write8<I4>(v, xb3 + 2 * t * K + 8 * i, K);
 }
 
-// One tile through `per` row blocks of BR = 64 TILES rows from rb0, columns 256 g0 .. 256 (g0 + ng) - 1.
+// One tile through one row block of BR = 64 TILES rows, columns 256 g0 .. 256 (g0 + ng) - 1.
 // Wave w owns TILES 16-row tiles of each of NM matrices per row block. src: the activation parts at the
 // tile's base row, so[q]: this thread's byte offset of staged row tid / 16 of block q, columns
-// 8 (tid % 16) ... emit(row block, acc) takes each finished row block: acc[t][q] of weight tile t
-// (matrix t / TILES) and accumulator block q. Uniform bases and 32-bit lane offsets keep the addresses
+// 8 (tid % 16) ... acc[t][q]: the sums of weight tile t (matrix t / TILES), accumulator block q. Uniform bases and 32-bit lane offsets keep the addresses
 // in scalar registers.
 //
 // A row's scales are fetched in lines (int4: 128 bytes, four groups; MXFP4: 64 bytes, eight), lane l
 // holding 1/4 of row l / 4's line: fetched a group's bytes at a time, the lines left the L2 between
 // their groups (0.5 GB more fetched at the shape above).
-template <bool I4, int NM, int TILES, int MODE, typename EMIT>
+template <bool I4, int NM, int TILES, int MODE>
 __device__ __forceinline__ void x3_run(const uint8_t *src, const uint32_t (&so)[x3_arows(MODE)],
-                                       const uint8_t *const (&a)[NM], const uint8_t *const (&sc)[NM], int K, int rb0,
-                                       int per, int g0, int ng, uint8_t *lds, EMIT emit) {
+                                       const uint8_t *const (&a)[NM], const uint8_t *const (&sc)[NM], int K, int rb,
+                                       int g0, int ng, uint8_t *lds, xf4 (&acc)[NM * TILES][MODE == X3_BIG ? 2 : 1]) {
   constexpr int NT = NM * TILES, BR = 64 * TILES, AR = x3_arows(MODE), NQ = MODE == X3_BIG ? 2 : 1;
   constexpr int NP = MODE == X3_SMALL ? 1 : 3;  // MFMAs chained per accumulator block
   constexpr int LG = I4 ? 4 : 8, GB = I4 ? 32 : 8, NL = I4 ? 2 : 1;  // groups per line, bytes per group, u4 per lane
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
-  const int total = per * ng;
-  if (total <= 0) return;  // uniform
   const int rowb = K >> 1, rows = I4 ? K >> 3 : K >> 5;  // bytes per row: codes, scales
   typedef __bf16 Buf[AR][16][X3_BS];
   Buf *bs = reinterpret_cast<Buf *>(lds);
@@ -170,36 +167,29 @@ __device__ __forceinline__ void x3_run(const uint8_t *src, const uint32_t (&so)[
   const uint8_t *pa[NT], *ps[NT];  // uniform
 #pragma unroll
   for (int t = 0; t < NT; t++) {
-    const long row = (long)rb0 * BR + 16 * TILES * w + 16 * (t % TILES);
+    const long row = (long)rb * BR + 16 * TILES * w + 16 * (t % TILES);
     pa[t] = a[t / TILES] + row * rowb + 128L * g0;
     ps[t] = sc[t / TILES] + row * rows + (long)GB * g0;
   }
   // codes: 8 rows x 128 bytes per instruction
   const uint32_t oc = (uint32_t)(lane >> 3) * rowb + 16 * (lane & 7);
-  int f_rb = 0, f_g = 0;  // next group to fetch (past the end: the last one again, never used)
+  int f_g = 0;  // next group to fetch (past the end: the last one again, never used)
   rbt_u4 nw[NT][2], ln[NT][NL];
   auto fetch = [&]() {
-    const int rb = min(f_rb, per - 1);
-    const int gg = f_rb < per ? f_g : ng - 1;
-    const long oa = (long)rb * BR * rowb + 128 * gg;
 #pragma unroll
     for (int q = 0; q < 2; q++)
 #pragma unroll
-      for (int t = 0; t < NT; t++) nw[t][q] = __builtin_nontemporal_load((const rbt_gu4 *)(pa[t] + oa + 8L * q * rowb + oc));
-    if (++f_g == ng) {
-      f_g = 0;
-      ++f_rb;
-    }
+      for (int t = 0; t < NT; t++) nw[t][q] = __builtin_nontemporal_load((const rbt_gu4 *)(pa[t] + 128L * f_g + 8L * q * rowb + oc));
+    f_g = min(f_g + 1, ng - 1);
   };
-  // line of groups LG l .. of row block rb: lane l's quarter, clamped to the last quarter in range
-  auto line = [&](int rb, int l) {
+  // line l (groups LG l ..): the lane's quarter, clamped to the last quarter in range
+  auto line = [&](int l) {
     const int q0 = LG / 4 * (4 * l + (lane & 3));  // first group of the quarter
     const uint32_t off = (uint32_t)(lane >> 2) * rows + GB * min(q0, ng - LG / 4);
-    const long ob = (long)rb * BR * rows;
 #pragma unroll
     for (int t = 0; t < NT; t++)
 #pragma unroll
-      for (int u = 0; u < NL; u++) ln[t][u] = *(const rbt_gu4 *)(ps[t] + ob + off + 16 * u);
+      for (int u = 0; u < NL; u++) ln[t][u] = *(const rbt_gu4 *)(ps[t] + off + 16 * u);
   };
   // activations: st[d] holds the next step of parity d, loaded a group ahead
   rbt_u4 st[2][AR];
@@ -208,7 +198,7 @@ __device__ __forceinline__ void x3_run(const uint8_t *src, const uint32_t (&so)[
   auto stage_load = [&](int slot) {
 #pragma unroll
     for (int q = 0; q < AR; q++) st[slot][q] = *(const rbt_gu4 *)(src + 256L * (2 * g0 + a_s) + so[q]);
-    if (++a_s == nst) a_s = 0;
+    a_s = min(a_s + 1, nst - 1);
   };
   const int tl = threadIdx.x >> 4, tc = threadIdx.x & 15;
   auto stage_store = [&](int slot) {
@@ -217,24 +207,23 @@ __device__ __forceinline__ void x3_run(const uint8_t *src, const uint32_t (&so)[
   };
   stage_load(0);
   stage_load(1);
-  line(0, 0);
+  line(0);
   fetch();
   stage_store(0);
   stage_load(0);
   __syncthreads();
   // ch: the chained products; cl (MXFP4, three chained parts): those of the two small parts, so that the
   // full-size sum rounds once per block and not three times
-  xf4 acc[NT][NQ], ch[NT][NQ], cl[NT][NQ];
+  xf4 ch[NT][NQ], cl[NT][NQ];
 #pragma unroll
   for (int t = 0; t < NT; t++)
 #pragma unroll
     for (int q = 0; q < NQ; q++) acc[t][q] = ch[t][q] = cl[t][q] = xf4{0.f, 0.f, 0.f, 0.f};
-  int c_rb = 0, c_g = 0;
-  for (int it = 0; it < total; it++) {
+  for (int it = 0; it < ng; it++) {
     // the group's codes -> the wave's LDS area; its scales: int4 from the lanes holding this quarter of
     // the line to LDS, MXFP4 by shuffles; then the next group's codes and, after a line's last group, the
     // next line
-    const int lq = c_g & (LG - 1);
+    const int lq = it & (LG - 1);
     uint2 cs[NT];
 #pragma unroll
     for (int t = 0; t < NT; t++) {
@@ -254,12 +243,7 @@ __device__ __forceinline__ void x3_run(const uint8_t *src, const uint32_t (&so)[
         cs[t].y = (uint32_t)__shfl((int)(lq & 1 ? v.w : v.y), from, 64);
       }
     }
-    if (lq == LG - 1 || c_g == ng - 1) {
-      if (c_g + 1 < ng)
-        line(c_rb, (c_g + 1) / LG);
-      else if (c_rb + 1 < per)
-        line(c_rb + 1, 0);
-    }
+    if (lq == LG - 1 && it + 1 < ng) line((it + 1) / LG);
     fetch();
 #pragma unroll
     for (int d = 0; d < 2; d++) {
@@ -320,15 +304,6 @@ __device__ __forceinline__ void x3_run(const uint8_t *src, const uint32_t (&so)[
           ch[t][q] = cl[t][q] = xf4{0.f, 0.f, 0.f, 0.f};
         }
     }
-    if (++c_g == ng) {  // row block done (uniform)
-      emit(rb0 + c_rb, acc);
-#pragma unroll
-      for (int t = 0; t < NT; t++)
-#pragma unroll
-        for (int q = 0; q < NQ; q++) acc[t][q] = xf4{0.f, 0.f, 0.f, 0.f};
-      c_g = 0;
-      ++c_rb;
-    }
   }
 }
 
@@ -375,7 +350,7 @@ __device__ __forceinline__ void x3_row(int q, int m, int &tok, int &part) {
 }
 
 template <bool I4, bool GATEUP, int MODE>
-__device__ __forceinline__ void x3_unit(const X3Args &A, const X3Tile &T, int KS, int ks, int rb0, uint8_t *lds) {
+__device__ __forceinline__ void x3_unit(const X3Args &A, const X3Tile &T, int KS, int ks, int rb, uint8_t *lds) {
   constexpr int NM = GATEUP ? 2 : 1, TILES = GATEUP ? 1 : 2, NT = NM * TILES, BR = 64 * TILES;
   constexpr int AR = x3_arows(MODE), NQ = MODE == X3_BIG ? 2 : 1;
   const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4, w = threadIdx.x >> 6;
@@ -400,49 +375,49 @@ __device__ __forceinline__ void x3_unit(const X3Args &A, const X3Tile &T, int KS
   } else {
     wa[0] = T.J.dd, ws[0] = (const uint8_t *)T.J.ds;
   }
-  x3_run<I4, NM, TILES, MODE>(src, so, wa, ws, K, rb0, 1, g0, g1 - g0, lds, [&](int rb, xf4(&acc)[NT][NQ]) {
-    const int o0 = rb * BR + 16 * TILES * w + r;
-    // v[t]: token tok's sum of weight tile t, row o0 + 16 (t % TILES)
-    auto put = [&](int tok, const float(&v)[NT]) {
-      if (tok >= T.M) return;
-      const long pr = T.pbase + tok;
-      if (A.part) {
+  xf4 acc[NT][NQ];
+  x3_run<I4, NM, TILES, MODE>(src, so, wa, ws, K, rb, g0, g1 - g0, lds, acc);
+  const int o0 = rb * BR + 16 * TILES * w + r;
+  // v[t]: token tok's sum of weight tile t, row o0 + 16 (t % TILES)
+  auto put = [&](int tok, const float(&v)[NT]) {
+    if (tok >= T.M) return;
+    const long pr = T.pbase + tok;
+    if (A.part) {
 #pragma unroll
-        for (int t = 0; t < NT; t++)
-          A.y[((long)(ks * NM + t / TILES) * T.n + pr) * O + o0 + 16 * (t % TILES)] = v[t];
-      } else if (GATEUP) {
-        __bf16 p[3];
-        x3_split(rbt_act(A.act, v[0], v[NT - 1]), p);
-        __bf16 *d = A.hb3 + 3 * pr * O + (o0 & ~7) + x3_pos(I4, o0 & 7);
+      for (int t = 0; t < NT; t++)
+        A.y[((long)(ks * NM + t / TILES) * T.n + pr) * O + o0 + 16 * (t % TILES)] = v[t];
+    } else if (GATEUP) {
+      __bf16 p[3];
+      x3_split(rbt_act(A.act, v[0], v[NT - 1]), p);
+      __bf16 *d = A.hb3 + 3 * pr * O + (o0 & ~7) + x3_pos(I4, o0 & 7);
 #pragma unroll
-        for (int q = 0; q < 3; q++) d[(long)q * O] = p[q];
-      } else {
-#pragma unroll
-        for (int t = 0; t < NT; t++) A.y[pr * O + o0 + 16 * t] = v[t];
-      }
-    };
-    if (MODE == X3_SMALL) {
-      float v[NT], v4[NT];
-#pragma unroll
-      for (int t = 0; t < NT; t++) {
-        v[t] = (acc[t][0][0] + acc[t][0][1]) + acc[t][0][2];
-        const float l = acc[t][0][3];
-        v4[t] = (__shfl(l, r, 64) + __shfl(l, 16 + r, 64)) + __shfl(l, 32 + r, 64);
-      }
-      put(g, v);
-      if (g == 0) put(4, v4);
+      for (int q = 0; q < 3; q++) d[(long)q * O] = p[q];
     } else {
 #pragma unroll
-      for (int q = 0; q < NQ; q++)
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-          float v[NT];
-#pragma unroll
-          for (int t = 0; t < NT; t++) v[t] = acc[t][q][i];
-          put(16 * q + 4 * g + i, v);
-        }
+      for (int t = 0; t < NT; t++) A.y[pr * O + o0 + 16 * t] = v[t];
     }
-  });
+  };
+  if (MODE == X3_SMALL) {
+    float v[NT], v4[NT];
+#pragma unroll
+    for (int t = 0; t < NT; t++) {
+      v[t] = (acc[t][0][0] + acc[t][0][1]) + acc[t][0][2];
+      const float l = acc[t][0][3];
+      v4[t] = (__shfl(l, r, 64) + __shfl(l, 16 + r, 64)) + __shfl(l, 32 + r, 64);
+    }
+    put(g, v);
+    if (g == 0) put(4, v4);
+  } else {
+#pragma unroll
+    for (int q = 0; q < NQ; q++)
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        float v[NT];
+#pragma unroll
+        for (int t = 0; t < NT; t++) v[t] = acc[t][q][i];
+        put(16 * q + 4 * g + i, v);
+      }
+  }
 }
 
 // Units (tile, row block, K part): XCD x (workgroups x, x + 8, ..) takes [x U / 8, (x + 1) U / 8), its
