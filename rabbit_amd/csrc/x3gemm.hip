@@ -564,9 +564,9 @@ hipError_t launch_x3split(const Ctx &c, int kind, const float *x, size_t S, size
 }
 
 hipError_t launch_x3(const Ctx &c, int kind, bool gateup, const X3Args &A) {
-  if (A.K % (2 * X3_KG) || A.O % (gateup ? 64 : 128) ) return hipErrorInvalidValue;
-
-  if ((A.tch != 16 && A.tch != 32) || 6L * A.S * A.K >= (1L << 32)) return hipErrorInvalidValue;
+  if (A.K % (2 * X3_KG) || A.O % (gateup ? 64 : 128) || (A.tch != 16 && A.tch != 32)) return hipErrorInvalidValue;
+  // a lane's 32-bit offset reaches over all S rows' parts through row_tok, else over one tile's
+  if (6L * (A.row_tok ? A.S : A.tch) * A.K >= (1L << 32)) return hipErrorInvalidValue;
   const dim3 grid(x3_wgs(c, A.tch)), blk(256);
 #define RBT_X3(I4_, GU_)                                                                   \
   {                                                                                        \

@@ -45,3 +45,14 @@ def ctx(rbt_lib):
     c = rabbit_amd.Context(0)
     yield c
     c.close()
+
+
+@pytest.fixture
+def own_ctx(rbt_lib):
+    """A context of the test's own: its scratch and layers go with it."""
+    import torch
+    import rabbit_amd as R
+    torch.zeros(1, device="cuda")
+    c = R.Context(0)
+    yield c
+    c.close()

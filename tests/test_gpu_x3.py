@@ -142,3 +142,67 @@ def test_grouping_past_the_lds_bitmaps(ctx, orc):
     ctx.moe_forward(0, x, S, out, ids, w)
     assert np.array_equal(ids.reshape(S, k), eids)
     assert rel_l2(out, exp) < 1e-2  # bf16 activations
+
+
+def _device_matrix(fmt, n, rows, cols, seed):
+    """n matrices on the device, codes and scales uniform, with their 64-bit values on demand."""
+    import torch
+    import rabbit_amd as R
+    g = torch.Generator(device="cuda")
+    g.manual_seed(seed)
+    data = torch.randint(0, 256, (n, rows, cols // 2), dtype=torch.uint8, device="cuda", generator=g)
+    if fmt == "mxfp4":
+        scale = torch.randint(119, 124, (n, rows, cols // 32), dtype=torch.uint8, device="cuda", generator=g)
+        return lambda e: R.QT.mxfp4(data[e], scale[e], rows, cols)
+    scale = torch.rand(n, rows, cols // 32, device="cuda", generator=g) * 0.015 + 0.005
+    return lambda e: R.QT.i4g(data[e], scale[e], rows, cols, 32)
+
+
+def _device_layer(ctx, fmt, H, I, E, k, shared, seed, layer=0, std=0.05):
+    """A layer of device-resident experts: {"gate"/"up"/"down": e -> QT (E: the shared expert)}."""
+    import torch
+    import rabbit_amd as R
+    m = {n: _device_matrix(fmt, E + 1, r, c, seed + i)
+         for i, (n, r, c) in enumerate((("gate", I, H), ("up", I, H), ("down", H, I)))}
+    slot = lambda e, eid: R.Slot(eid, m["down"](e), gate=m["gate"](e), up=m["up"](e))  # noqa: E731
+    for e in range(E):
+        ctx.pool_put(layer, slot(e, e))
+    router = torch.from_numpy(normal((E, H), seed + 9, std)).cuda()
+    ctx.moe_layer_set(layer, R.FAMILY_GLM52, H, I, E, k, router, shared=slot(E, 0) if shared else None)
+    return m
+
+
+def _ffn64(ctx, m, e, x):
+    """down(silu(gate x) * up x) of one expert in 64 bits, the weights dequantized."""
+    import torch
+    w = {n: ctx.dequant_rows(f(e), 0, f(e).rows).reshape(f(e).rows, f(e).cols).double() for n, f in m.items()}
+    return (torch.nn.functional.silu(x @ w["gate"].t()) * (x @ w["up"].t())) @ w["down"].t()
+
+
+def test_int4_layer_many_tokens_wide_experts(own_ctx):
+    """More than 2^32 bytes of the down product's activation parts (6 * tokens * inter): the offsets a lane
+    holds in 32 bits reach over one tile there, so the call's size does not bound them. Checked at the first and
+    last tokens of the call and of each expert's tiles."""
+    import torch
+    ctx = own_ctx
+    H, I, E, k, S = 512, 65536, 2, 1, 10945
+    m = _device_layer(ctx, "i4g", H, I, E, k, True, 300)
+    g = torch.Generator(device="cuda")
+    g.manual_seed(3)
+    x = torch.randn(S, H, device="cuda", generator=g)
+    out = torch.empty(S, H, device="cuda")
+    ids, w = torch.empty(S, k, dtype=torch.int32, device="cuda"), torch.empty(S, k, device="cuda")
+    ctx.moe_forward(0, x, S, out, ids, w)
+    picked = set(range(4)) | set(range(S - 4, S))
+    for e in range(E):
+        t = torch.nonzero(ids[:, 0] == e).flatten().tolist()
+        assert len(t) > 100
+        picked |= {t[0], t[15], t[16], t[31], t[32], t[-2], t[-1]}
+    rows = torch.tensor(sorted(picked), device="cuda")
+    xr = x[rows].double()
+    want = _ffn64(ctx, m, E, xr)
+    for e in range(E):
+        at = torch.nonzero(ids[rows, 0] == e).flatten()
+        want[at] += w[rows[at], 0].double()[:, None] * _ffn64(ctx, m, e, xr[at])
+    err = (out[rows].double() - want).norm(dim=1) / want.norm(dim=1)
+    assert float(err.max()) < 1e-5, err
