@@ -913,21 +913,23 @@ int x3_experts(rbt_ctx *c, int kind, const RbtExpertDev *table, const RbtExpertD
 // Router logits and selection of a call (not the one-token fused launches): a decode batch as certified
 // intervals for every (row, token) with a selection workgroup per token (whose idle waves write xb3_sel,
 // the tokens' three-part split, when given); larger batches on the matrix cores with a rigorous bound on
-// the distance to the reference's sequential fp32 fold, or as that fold itself.
+// the distance to the reference's sequential fp32 fold, or as that fold itself. Below 64 tokens the
+// matrix-core logits' scratch is `spare` (spare_n floats: the layer's expert rows, written later), so that
+// the choice depends on the shape alone and takes no memory the call's later buffers need.
 int route_logits_select(rbt_ctx *c, const rbt::RouterArgs &ra, int erows, const float *sgate, const RbtExpertDev *table,
                         double *mid, double *bnd, int32_t *ids, float *wts, float *shs, const rbt::GroupArgs *ga,
-                        const rbt::SharedGateUp *sgu, __bf16 *xb3_sel) {
+                        const rbt::SharedGateUp *sgu, __bf16 *xb3_sel, float *spare, size_t spare_n) {
   int *amb = c->d_flags + FLAG_AMB;
   const bool al = al16({ra.x, ra.W, sgate});
   const bool bounded = ra.S >= rbt::RB_MIN_S && rbt::router_bounded_ok(ra) && al &&
-                       (ra.S >= 64 || scratch_avail(c, {{SC_RLOG, rbt::router_bounded_scratch(ra, erows)}}));
+                       (ra.S >= 64 || rbt::router_bounded_scratch(ra, erows) <= 4 * spare_n);
   if (!bounded && !rbt::router_exact_ok(ra.S, ra.H) && rbt::router_batch_ok(ra) && al16({sgate})) {
     HIP_OK(c, rbt::launch_router_batch(*c, ra, sgate, mid, bnd, table, ids, wts, shs, amb, xb3_sel));
     return RBT_OK;
   }
   if (bounded) {
-    void *rs;
-    RBT_TRY(scratch(c, SC_RLOG, rbt::router_bounded_scratch(ra, erows), &rs));
+    void *rs = spare;
+    if (ra.S >= 64) RBT_TRY(scratch(c, SC_RLOG, rbt::router_bounded_scratch(ra, erows), &rs));
     HIP_OK(c, rbt::launch_router_bounded(*c, ra, sgate, mid, bnd, rs));
   } else if (rbt::router_exact_ok(ra.S, ra.H) && al) {
     float *lg;
@@ -1092,7 +1094,7 @@ int moe_forward_dev(rbt_ctx *c, uint32_t layer, const float *x, size_t s, float 
     if (dgrouped && !rbt::router_exact_ok(S, H) && rbt::router_batch_ok(ra) && al16({sgate, x}) && H % 4 == 0)
       RBT_TRY(scratch_t(c, SC_XB, (size_t)3 * S * H, &xb3_sel));
     RBT_TRY(route_logits_select(c, ra, erows, sgate, L.d_table, mid, bnd, ids, wts, shs, grp_in_select ? &ga : nullptr,
-                                sh_in_select ? &sgu : nullptr, xb3_sel));
+                                sh_in_select ? &sgu : nullptr, xb3_sel, yy, (size_t)npairs * H));
   }
   const bool grouped = !dgrouped && !mfma && S > 1 && (merge || !D.has_shared) &&
                        rbt::prefill_ok(L.routed_kind, H, I, (size_t)E, (size_t)k);
@@ -1401,7 +1403,7 @@ static int latent_moe_dev(rbt_ctx *c, uint32_t layer, const rbt_latent_moe_desc 
                                            (int)H, (int)MH, xl));
   } else {
     RBT_TRY(route_logits_select(c, ra, (int)E, nullptr, table, mid, bnd, ids, wts, shs, grp_in_select ? &ga : nullptr,
-                                nullptr, nullptr));
+                                nullptr, nullptr, yy, (size_t)P * MH));
     RBT_TRY(matmul_dev(c, xl, x, &lw->down_proj, s));
   }
   if (x3_experts_ok(c, kind, gs, Ly.lat_al16, xl, S, K, (int)E, (int)MH, (int)I, 0)) {

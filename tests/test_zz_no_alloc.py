@@ -62,3 +62,17 @@ def test_noalloc_small_layers(ctx, orc):
         for S in (6, 1):
             print(f"noalloc family={family} S={S}", flush=True)
             _check(ctx, x[:S].contiguous(), S, H, k)
+
+
+# the last token counts whose buffers fit the fixed array
+@pytest.mark.parametrize("name,counts", [("c1", (26, 27, 28, 29)), ("c3", (35, 36, 37))])
+def test_noalloc_short_prompts(own_ctx, name, counts):
+    """A prompt of 17 to 63 tokens: nothing the router may use is taken from what the experts need."""
+    import torch
+    import rabbit_amd.workloads as W
+    cfg = W.CONFIGS[name]
+    W.build_layer(own_ctx, cfg, layer=0, seed=1100)
+    x = torch.from_numpy(W.tokens(cfg, max(counts), 33)).cuda()
+    for S in counts:
+        print(f"noalloc {name} S={S}", flush=True)
+        _check(own_ctx, x[:S].contiguous(), S, cfg.hidden, cfg.topk)
