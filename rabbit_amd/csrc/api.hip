@@ -939,7 +939,14 @@ int route_logits_select(rbt_ctx *c, const rbt::RouterArgs &ra, int erows, const 
   } else {
     HIP_OK(c, rbt::launch_router_logits(*c, ra.x, ra.S, ra.H, ra.W, ra.E, sgate, mid, bnd));
   }
-  HIP_OK(c, rbt::launch_router_select(*c, ra, mid, bnd, ids, wts, shs, amb, ga, sgu));
+  // The matrix cores sum 32 products in fp32 before the fp64 sum, the certified form rounds each product
+  // once: softmax weights of 37 tokens (hidden 4096, 512 experts) are 4.9e-7 from 64 bits with the former's
+  // midpoints, 2.1e-7 with the latter's and 1.4e-7 with the winners' logits summed again, which costs 8 us
+  // of 1372 (hidden 8192, top-10).
+  rbt::RouterArgs sel = ra;
+  sel.refine = bounded && ra.S < 64;
+  sel.sgate = sgate;
+  HIP_OK(c, rbt::launch_router_select(*c, sel, mid, bnd, ids, wts, shs, amb, ga, sgu));
   return RBT_OK;
 }
 

@@ -57,6 +57,10 @@ struct RouterArgs {
   float routed_scale;
   int n_group, topk_group;
   const float *x, *W;
+  // launch_router_select: weights from the winners' logits (and sgate's) summed again in 64 bits; x, W and
+  // sgate 16-byte aligned, H a multiple of 4, no expert groups
+  bool refine = false;
+  const float *sgate = nullptr;
 };
 
 // shards.hip: base names, shapes and the packed tensor's suffix of one MXFP4 expert's three

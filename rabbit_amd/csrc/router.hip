@@ -455,6 +455,7 @@ struct SelParams {
   int n_group, topk_group;
   const float *x;  // [S, H] for exact recomputation
   const float *W;  // [E, H]
+  const float *sgate = nullptr;  // REFINE: the shared-expert gate row [H], or null
 };
 
 // Selection key of one logit value for the family (monotone non-decreasing in the logit).
@@ -750,6 +751,33 @@ __device__ float exact_logit_wave(const float *__restrict__ xs, const float *__r
 }
 
 
+// sum of x[i] w[i] in 64 bits (products exact) by one wave, in every lane. Rows 16-byte aligned, H a
+// multiple of 4; eight 16-byte loads of each row in flight per lane.
+__device__ double logit_wave_f64(const float *__restrict__ xs, const float *__restrict__ w, int H) {
+  const int lane = threadIdx.x & 63, H4 = H >> 2;
+  const float4 *x4 = reinterpret_cast<const float4 *>(xs);
+  const float4 *w4 = reinterpret_cast<const float4 *>(w);
+  double a = 0.0, b = 0.0;
+  for (int base = 0; base < H4; base += 512) {
+    float4 xv[8], wv[8];
+#pragma unroll
+    for (int j = 0; j < 8; j++) {
+      const int i = min(base + 64 * j + lane, H4 - 1);
+      xv[j] = x4[i];
+      wv[j] = w4[i];
+    }
+#pragma unroll
+    for (int j = 0; j < 8; j++)
+      if (base + 64 * j + lane < H4) {
+        a = fma((double)xv[j].x, (double)wv[j].x, a);
+        b = fma((double)xv[j].y, (double)wv[j].y, b);
+        a = fma((double)xv[j].z, (double)wv[j].z, a);
+        b = fma((double)xv[j].w, (double)wv[j].w, b);
+      }
+  }
+  return rbt_wave_total_d(a + b);
+}
+
 // The same fold with the serial chain on one lane, for a wave that has a 2 x 1024-float LDS buffer
 // of its own: the wave forms the products of 1024-element blocks in parallel into the buffer, in
 // element order, and lane 0 walks the previous block with 16-byte LDS reads (two groups of eight in
@@ -964,7 +992,9 @@ __device__ __forceinline__ void sel_keys(const SelParams &P, double mv, double b
 // MW: the keys of all experts are computed by the four waves together (for the sigmoid families
 // each key costs three fp64-exp sigmoids) and handed to wave 0 through kbuf, LDS of 4 * 64 * MAXM
 // words; otherwise wave 0 computes them alone and kbuf is unused.
-template <int MAXM, bool MW = false>
+// REFINE: the weights come from the winners' logits (and the shared gate's) summed again in 64 bits, for
+// midpoints whose products were partly summed in fp32 (k_rcert).
+template <int MAXM, bool MW = false, bool REFINE = false>
 __device__ __forceinline__ void select3_body(SelLds &L, const SelParams &P, const double *__restrict__ mid,
                                              const double *__restrict__ bnd, int32_t *__restrict__ ids,
                                              float *__restrict__ wts, float *__restrict__ sh_scale,
@@ -1278,6 +1308,18 @@ __device__ __forceinline__ void select3_body(SelLds &L, const SelParams &P, cons
     }
     __syncthreads();
   }
+  double gate_mid = P.erows > E ? ms[E] : 0.0;
+  if constexpr (REFINE) {
+    for (int r = wave; r < kk; r += 4) {
+      const float l = (float)logit_wave_f64(P.x + (size_t)s * P.H, P.W + (size_t)r_id[r] * P.H, P.H);
+      if (lane == 0 && isfinite(l)) r_l[r] = l;  // (not finite: the fold's own value stays)
+    }
+    if (wave == 0 && P.sgate) {
+      const double g = logit_wave_f64(P.x + (size_t)s * P.H, P.sgate, P.H);
+      if (isfinite(g)) gate_mid = g;
+    }
+    __syncthreads();
+  }
   if (wave == 0) {
     if (lane == 0 && stats && total_amb) atomicAdd(stats, total_amb);
     winner_weights(L, P, kk);
@@ -1287,7 +1329,7 @@ __device__ __forceinline__ void select3_body(SelLds &L, const SelParams &P, cons
       io[r] = r < kk ? r_id[r] : -1;
       wo[r] = r < kk ? s_w[r] : 0.0f;
     }
-    if (lane == 0 && sh_scale) sh_scale[s] = (P.erows > E) ? sigmoid_ref(__double2float_rn(ms[E])) : 1.0f;
+    if (lane == 0 && sh_scale) sh_scale[s] = (P.erows > E) ? sigmoid_ref(__double2float_rn(gate_mid)) : 1.0f;
     if (grp) {
       // single token: pair j = slot j; the shared expert is at G.shared_slot
       auto put = [&](int r, const uint8_t *gd, const void *gs, const uint8_t *ud, const void *us, const uint8_t *dd,
@@ -1343,14 +1385,14 @@ __device__ __forceinline__ void select3_body(SelLds &L, const SelParams &P, cons
   }
 }
 
-template <int MAXM>
+template <int MAXM, bool REFINE>
 __global__ __launch_bounds__(256) void k_router_select3(SelParams P, const double *__restrict__ mid,
                                                         const double *__restrict__ bnd, int32_t *__restrict__ ids,
                                                         float *__restrict__ wts, float *__restrict__ sh_scale,
                                                         int *__restrict__ stats, GroupOut G, int grp) {
   __shared__ SelLds L;
   __shared__ float kbuf[6 * 64 * MAXM];
-  select3_body<MAXM, true>(L, P, mid, bnd, ids, wts, sh_scale, stats, G, grp, blockIdx.x, kbuf);
+  select3_body<MAXM, true, REFINE>(L, P, mid, bnd, ids, wts, sh_scale, stats, G, grp, blockIdx.x, kbuf);
 }
 
 // One token with a shared expert: workgroup 0 selects; the other workgroups stream the shared
@@ -1876,6 +1918,7 @@ hipError_t launch_router_select(const Ctx &c, const RouterArgs &a, const double 
   P.topk_group = a.topk_group;
   P.x = a.x;
   P.W = a.W;
+  P.sgate = a.sgate;
   if (a.n_group > 1 && a.family != RBT_FAMILY_QWEN38) {
     launch_k(c, k_router_select_grouped, dim3(a.S), dim3(64), P, mid, bnd, ids, wts, sh_scale,
                        stats);
@@ -1907,18 +1950,18 @@ hipError_t launch_router_select(const Ctx &c, const RouterArgs &a, const double 
       return hipGetLastError();
     }
     if (sgu) return hipErrorInvalidValue;
+#define RBT_SEL3(M_)                                                                                               \
+  launch_k(c, a.refine ? k_router_select3<M_, true> : k_router_select3<M_, false>, dim3(a.S), dim3(256), P, mid, bnd, \
+           ids, wts, sh_scale, stats, G, g)
     if (m <= 4)
-      launch_k(c, k_router_select3<4>, dim3(a.S), dim3(256), P, mid, bnd, ids, wts, sh_scale, stats,
-                         G, g);
+      RBT_SEL3(4);
     else if (m <= 8)
-      launch_k(c, k_router_select3<8>, dim3(a.S), dim3(256), P, mid, bnd, ids, wts, sh_scale, stats,
-                         G, g);
+      RBT_SEL3(8);
     else if (m <= 16)
-      launch_k(c, k_router_select3<16>, dim3(a.S), dim3(256), P, mid, bnd, ids, wts, sh_scale,
-                         stats, G, g);
+      RBT_SEL3(16);
     else
-      launch_k(c, k_router_select3<32>, dim3(a.S), dim3(256), P, mid, bnd, ids, wts, sh_scale,
-                         stats, G, g);
+      RBT_SEL3(32);
+#undef RBT_SEL3
   }
   return hipGetLastError();
 }

@@ -158,8 +158,8 @@ def _device_matrix(fmt, n, rows, cols, seed):
     return lambda e: R.QT.i4g(data[e], scale[e], rows, cols, 32)
 
 
-def _device_layer(ctx, fmt, H, I, E, k, shared, seed, layer=0, std=0.05):
-    """A layer of device-resident experts: {"gate"/"up"/"down": e -> QT (E: the shared expert)}."""
+def _device_layer(ctx, fmt, H, I, E, k, shared, seed, layer=0, std=0.05, family=1, gated=False):
+    """A layer of device-resident experts: {"gate"/"up"/"down": e -> QT (E: the shared expert), "router"}."""
     import torch
     import rabbit_amd as R
     m = {n: _device_matrix(fmt, E + 1, r, c, seed + i)
@@ -168,8 +168,9 @@ def _device_layer(ctx, fmt, H, I, E, k, shared, seed, layer=0, std=0.05):
     for e in range(E):
         ctx.pool_put(layer, slot(e, e))
     router = torch.from_numpy(normal((E, H), seed + 9, std)).cuda()
-    ctx.moe_layer_set(layer, R.FAMILY_GLM52, H, I, E, k, router, shared=slot(E, 0) if shared else None)
-    return m
+    gate = torch.from_numpy(normal(H, seed + 8, std)).cuda() if gated else None
+    ctx.moe_layer_set(layer, family, H, I, E, k, router, shared=slot(E, 0) if shared else None, shared_gate=gate)
+    return m, router
 
 
 def _ffn64(ctx, m, e, x):
@@ -186,7 +187,7 @@ def test_int4_layer_many_tokens_wide_experts(own_ctx):
     import torch
     ctx = own_ctx
     H, I, E, k, S = 512, 65536, 2, 1, 10945
-    m = _device_layer(ctx, "i4g", H, I, E, k, True, 300)
+    m, _ = _device_layer(ctx, "i4g", H, I, E, k, True, 300)
     g = torch.Generator(device="cuda")
     g.manual_seed(3)
     x = torch.randn(S, H, device="cuda", generator=g)
@@ -206,3 +207,30 @@ def test_int4_layer_many_tokens_wide_experts(own_ctx):
         want[at] += w[rows[at], 0].double()[:, None] * _ffn64(ctx, m, e, xr[at])
     err = (out[rows].double() - want).norm(dim=1) / want.norm(dim=1)
     assert float(err.max()) < 1e-5, err
+
+
+@pytest.mark.parametrize("family", [0, 1])
+def test_routing_weights_of_short_prompts(own_ctx, family):
+    """The routing weights of 37 tokens (router logits on the matrix cores) are no further from 64 bits than
+    those of the same tokens in calls of at most 16 (certified logits), and name the same experts."""
+    import torch
+    H, I, E, k, S = 4096, 1024, 512, 10, 37
+    _, router = _device_layer(own_ctx, "mxfp4", H, I, E, k, True, 500, std=0.03, family=family, gated=family == 0)
+    x = torch.from_numpy(normal((S, H), 41)).cuda()
+
+    def call(t):
+        n = t.shape[0]
+        out = torch.empty(n, H, device="cuda")
+        ids, w = torch.empty(n, k, dtype=torch.int32, device="cuda"), torch.empty(n, k, device="cuda")
+        own_ctx.moe_forward(0, t, n, out, ids, w)
+        return ids, w
+
+    ids, w = call(x)
+    small = [call(x[a:a + 16].contiguous()) for a in range(0, S, 16)]
+    assert bool((ids == torch.cat([i for i, _ in small])).all())
+    logits = torch.gather(x.double() @ router.double().t(), 1, ids.long())
+    p = torch.softmax(logits, dim=1) if family == 0 else torch.sigmoid(logits)
+    want = p if family == 0 else p / (p.sum(1, keepdim=True) + 1e-20)
+    err = [float((v.double() - want).norm() / want.norm()) for v in (w, torch.cat([v for _, v in small]))]
+    print("error against 64 bits: one call", err[0], "small calls", err[1])
+    assert err[0] <= err[1], err
