@@ -910,6 +910,15 @@ int x3_experts(rbt_ctx *c, int kind, const RbtExpertDev *table, const RbtExpertD
   return RBT_OK;
 }
 
+// Tokens times experts from which calls of 17 to 63 tokens take the matrix-core logits (two launches and
+// the general selection, 64-row tiles) rather than one workgroup per (row, token) with the batch selection.
+// A layer of small MXFP4 experts, us, certified against matrix cores: 8192 x 16 experts 32 tokens 93 / 126;
+// 8192 x 128 40 tokens 282 / 297, 63 387 / 385; 8192 x 256 32 tokens 333 / 336, 40 405 / 393, 63 557 / 523;
+// 7168 x 512 20 tokens 294 / 281, 63 633 / 540; 2048 x 256 32 tokens 126 / 121. Where the batch form does
+// not apply (hidden no multiple of 1024) the certified logits read a row on one wave: 3584 x 128 17 tokens
+// 164 / 116, 63 407 / 191, and the matrix cores take all of them.
+constexpr long RB_LINE = 10000;
+
 // Router logits and selection of a call (not the one-token fused launches): a decode batch as certified
 // intervals for every (row, token) with a selection workgroup per token (whose idle waves write xb3_sel,
 // the tokens' three-part split, when given); larger batches on the matrix cores with a rigorous bound on
@@ -920,10 +929,12 @@ int route_logits_select(rbt_ctx *c, const rbt::RouterArgs &ra, int erows, const 
                         double *mid, double *bnd, int32_t *ids, float *wts, float *shs, const rbt::GroupArgs *ga,
                         const rbt::SharedGateUp *sgu, __bf16 *xb3_sel, float *spare, size_t spare_n) {
   int *amb = c->d_flags + FLAG_AMB;
-  const bool al = al16({ra.x, ra.W, sgate});
+  const bool al = al16({ra.x, ra.W, sgate}), exact = rbt::router_exact_ok(ra.S, ra.H);
+  const bool batch = !exact && rbt::router_batch_ok(ra) && al16({sgate});
   const bool bounded = ra.S >= rbt::RB_MIN_S && rbt::router_bounded_ok(ra) && al &&
+                       (exact || !batch || (long)ra.S * ra.E >= RB_LINE) &&
                        (ra.S >= 64 || rbt::router_bounded_scratch(ra, erows) <= 4 * spare_n);
-  if (!bounded && !rbt::router_exact_ok(ra.S, ra.H) && rbt::router_batch_ok(ra) && al16({sgate})) {
+  if (batch && !bounded) {
     HIP_OK(c, rbt::launch_router_batch(*c, ra, sgate, mid, bnd, table, ids, wts, shs, amb, xb3_sel));
     return RBT_OK;
   }
@@ -931,7 +942,7 @@ int route_logits_select(rbt_ctx *c, const rbt::RouterArgs &ra, int erows, const 
     void *rs = spare;
     if (ra.S >= 64) RBT_TRY(scratch(c, SC_RLOG, rbt::router_bounded_scratch(ra, erows), &rs));
     HIP_OK(c, rbt::launch_router_bounded(*c, ra, sgate, mid, bnd, rs));
-  } else if (rbt::router_exact_ok(ra.S, ra.H) && al) {
+  } else if (exact && al) {
     float *lg;
     RBT_TRY(scratch_t(c, SC_RLOG, (size_t)ra.S * erows, &lg));
     HIP_OK(c, rbt::launch_router_logits_exact(*c, ra.x, ra.S, ra.H, ra.W, ra.E, sgate, lg));

@@ -234,3 +234,18 @@ def test_routing_weights_of_short_prompts(own_ctx, family):
     err = [float((v.double() - want).norm() / want.norm()) for v in (w, torch.cat([v for _, v in small]))]
     print("error against 64 bits: one call", err[0], "small calls", err[1])
     assert err[0] <= err[1], err
+
+
+@pytest.mark.parametrize("H,E,S,cores", [(1024, 16, 63, False), (2048, 160, 62, False), (2048, 160, 63, True),
+                                           (512, 16, 17, True)])
+def test_router_of_short_prompts(own_ctx, H, E, S, cores):
+    """Few tokens times experts keep the certified logits (the matrix cores' were up to half slower there)."""
+    import torch
+    I, k = 1024, 4
+    _device_layer(own_ctx, "mxfp4", H, I, E, k, False, 600)
+    x, out = torch.from_numpy(normal((S, H), 3)).cuda(), torch.empty(S, H, device="cuda")
+    own_ctx.profile_kernels()
+    own_ctx.moe_forward(0, x, S, out)
+    names = " ".join(own_ctx.profile_kernels_read())
+    own_ctx.profile_kernels(False)
+    assert ("k_rcert" in names) == cores, names
