@@ -1840,10 +1840,11 @@ __global__ __launch_bounds__(256) void k_rcomb(const RbRec *__restrict__ part, i
   bnd[idx] = B;
 }
 
-static int router_bounded_ks(const RouterArgs &a, int erows) {
+static int router_bounded_ks(const RouterArgs &a, int erows, size_t bytes) {
   const long tiles = (long)((a.S + RB_WGT - 1) / RB_WGT) * ((erows + RB_WGT - 1) / RB_WGT);
   int ks = 8;
   while (ks > 1 && (tiles * 4 * (ks / 2) >= 2048 || a.H % (2 * RB_STEP * ks) != 0)) ks /= 2;
+  while (ks > 1 && (size_t)ks * a.S * erows * sizeof(RbRec) > bytes) ks /= 2;  // fewer parts where they have to fit
   return ks;
 }
 
@@ -1851,16 +1852,16 @@ bool router_bounded_ok(const RouterArgs &a) {
   return a.S >= 1 && a.E >= 1 && a.H % (2 * RB_STEP) == 0 && a.H > 0 && a.n_group <= 1;
 }
 
-size_t router_bounded_scratch(const RouterArgs &a, int erows) {
-  return (size_t)router_bounded_ks(a, erows) * a.S * erows * sizeof(RbRec);
+size_t router_bounded_scratch(const RouterArgs &a, int erows, size_t bytes) {
+  return (size_t)router_bounded_ks(a, erows, bytes) * a.S * erows * sizeof(RbRec);
 }
 
 hipError_t launch_router_bounded(const Ctx &c, const RouterArgs &a, const float *sgate, double *mid, double *bnd,
-                                 void *scratch) {
+                                 void *scratch, size_t bytes) {
   const int erows = a.E + (sgate ? 1 : 0);
-  if (!router_bounded_ok(a)) return hipErrorInvalidValue;
+  if (!router_bounded_ok(a) || router_bounded_scratch(a, erows, bytes) > bytes) return hipErrorInvalidValue;
   if (((uintptr_t)a.x | (uintptr_t)a.W | (uintptr_t)(sgate ? sgate : a.x)) % 16 != 0) return hipErrorInvalidValue;
-  const int ks = router_bounded_ks(a, erows);
+  const int ks = router_bounded_ks(a, erows, bytes);
   const int n_t = (a.S + RB_WGT - 1) / RB_WGT, n_e = (erows + RB_WGT - 1) / RB_WGT;
   const int nwg = n_t * n_e * ks, run = (nwg + 7) / 8;
   RbRec *part = static_cast<RbRec *>(scratch);

@@ -237,7 +237,7 @@ def test_routing_weights_of_short_prompts(own_ctx, family):
 
 
 @pytest.mark.parametrize("H,E,S,cores", [(1024, 16, 63, False), (2048, 160, 62, False), (2048, 160, 63, True),
-                                           (512, 16, 17, True)])
+                                           (512, 16, 17, True), (512, 512, 17, True), (576, 40, 70, True)])
 def test_router_of_short_prompts(own_ctx, H, E, S, cores):
     """Few tokens times experts keep the certified logits (the matrix cores' were up to half slower there)."""
     import torch
@@ -249,3 +249,8 @@ def test_router_of_short_prompts(own_ctx, H, E, S, cores):
     names = " ".join(own_ctx.profile_kernels_read())
     own_ctx.profile_kernels(False)
     assert ("k_rcert" in names) == cores, names
+    ids, one = (torch.empty(n, k, dtype=torch.int32, device="cuda") for n in (S, 1))
+    own_ctx.moe_forward(0, x, S, out, ids)
+    for t in range(0, S, 8):
+        own_ctx.moe_forward(0, x[t:t + 1].contiguous(), 1, out, one)
+        assert bool((ids[t] == one[0]).all()), t
