@@ -839,39 +839,55 @@ size_t group_scratch(int S, int E, long max_tiles, size_t (&off)[4]) {
   return off[3] + 256;
 }
 
-bool x3_experts_ok(rbt_ctx *c, int kind, size_t gs, bool aligned, const float *x, int S, int k, int E, int H, int I,
-                   int has_shared) {
+// Where the tiled products keep what they need beside the pairs' rows: nothing of their own, so that the
+// choice depends on the shape alone and a call runs the same kernels whatever memory there is. `area` starts
+// with the rows yy (written by the down launch, last) and ends with the GEMVs' h. The activations' parts lie
+// at its start (dead once gate/up has run), h's parts at its end, the grouping between them.
+struct X3Area {
+  size_t grp = 0, hb3 = 0;  // byte offsets
+  bool fits = false;
+};
+X3Area x3_area(int S, int k, int E, int H, int I, int has_shared, size_t area) {
+  const size_t pairs = (size_t)S * (k + has_shared), hb3 = 6 * pairs * I;
   size_t off[4];
+  X3Area a;
+  a.grp = align256(std::max((size_t)6 * S * H, 4 * pairs * H));
+  const size_t end = a.grp + group_scratch(S, E, rbt::x3_max_tiles(S, k, E, has_shared, 16), off);
+  a.fits = end + hb3 + 255 <= area;
+  if (a.fits) a.hb3 = (area - hb3) & ~(size_t)255;
+  return a;
+}
+
+bool x3_experts_ok(rbt_ctx *c, int kind, size_t gs, bool aligned, const float *x, int S, int k, int E, int H, int I,
+                   int has_shared, size_t area) {
   // The tiled products stream each unique expert once, the GEMVs once per (token, expert) pair and
   // somewhat faster. int4, hidden 6144, top-8 of 256 and a shared expert, us, GEMV against tiled: 4 tokens
   // 197 / 203, 6 271 / 289, 8 345 / 333, 16 650 / 572, 40 1553 / 952: the line lies where the pairs are
   // 1.22 times the experts that uniform routing picks. MXFP4 (moe_hidden 3584 x 3072, top-16 of 896):
   // 4 tokens 320 / 336, 8 552 / 514, 16 970 / 834, 131 6.9 ms / 2.5 ms: 1.06 times.
   const double uniq = E * (1.0 - std::pow(1.0 - std::min(1.0, (double)k / E), S)) + has_shared;
-  return S >= 2 && (double)S * (k + has_shared) >= (kind == RBT_QT_I4_GROUPED ? 1.22 : 1.06) * uniq && aligned && al16({x}) && (size_t)6 * S * H < ((size_t)1 << 32) &&
-         rbt::x3_ok(kind, gs, H, I, true) &&
+  return S >= 2 && (double)S * (k + has_shared) >= (kind == RBT_QT_I4_GROUPED ? 1.22 : 1.06) * uniq && aligned &&
+         al16({x}) && (size_t)6 * S * H < ((size_t)1 << 32) && rbt::x3_ok(kind, gs, H, I, true) &&
          rbt::x3_ok(kind, gs, I, H, false) && E + 1 <= rbt::PG_MAXE &&
-         scratch_avail(c, {{SC_PGRP, group_scratch(S, E, rbt::x3_max_tiles(S, k, E, has_shared, 16), off)},
-                           {SC_XB, (size_t)6 * S * H}});
+         x3_area(S, k, E, H, I, has_shared, area).fits;
 }
 
 // A batch through its routed (and shared) experts with fp32 accuracy, every unique expert's weights
 // streamed once per tile of its tokens: grouping, the activations' exact parts, gate/up with the
-// activation, down. yy [pairs, H] gets the pairs' rows in launch_pgroup's order, tpair / tw what
-// launch_combine needs. h: 2 I floats per pair.
+// activation, down. yy [pairs, H], the start of `area` bytes, gets the pairs' rows in launch_pgroup's order,
+// tpair / tw what launch_combine needs.
 int x3_experts(rbt_ctx *c, int kind, const RbtExpertDev *table, const RbtExpertDev *shared_dev, int has_shared,
                const float *x, int S, int k, int E, int H, int I, const int32_t *ids, const float *wts, int *ptok,
-               int *tpair, float *tw, float *h, float *yy, const RbtAct &act, hipEvent_t *ev) {
+               int *tpair, float *tw, float *yy, size_t area, const RbtAct &act, hipEvent_t *ev) {
   const int tch = x3_tch((size_t)S * k / E);
+  const X3Area at = x3_area(S, k, E, H, I, has_shared, area);
   size_t off[4];
-  void *blk;
-  RBT_TRY(scratch(c, SC_PGRP, group_scratch(S, E, rbt::x3_max_tiles(S, k, E, has_shared, 16), off), &blk));
-  char *b = static_cast<char *>(blk);
+  group_scratch(S, E, rbt::x3_max_tiles(S, k, E, has_shared, 16), off);
+  char *b = reinterpret_cast<char *>(yy) + at.grp;
   rbt::PSeg *segs = reinterpret_cast<rbt::PSeg *>(b + off[1]);
   rbt::PTile *tiles = reinterpret_cast<rbt::PTile *>(b + off[2]);
   int *ntiles = reinterpret_cast<int *>(b + off[3]);
-  __bf16 *xb3;
-  RBT_TRY(scratch_t(c, SC_XB, (size_t)3 * S * H, &xb3));
+  __bf16 *xb3 = reinterpret_cast<__bf16 *>(yy);  // [3 S, H]
   int *dflags = c->d_flags;
   HIP_OK(c, rbt::launch_pgroup(*c, ids, wts, S, k, E, has_shared, table, reinterpret_cast<uint32_t *>(b),
                                reinterpret_cast<uint32_t *>(b + off[0]), segs, tiles, ntiles, ptok, tpair, tw,
@@ -889,7 +905,7 @@ int x3_experts(rbt_ctx *c, int kind, const RbtExpertDev *table, const RbtExpertD
   A.xb3 = xb3;
   A.K = H;
   A.O = I;
-  A.hb3 = reinterpret_cast<__bf16 *>(h);  // [3 pairs, I]
+  A.hb3 = reinterpret_cast<__bf16 *>(reinterpret_cast<char *>(yy) + at.hb3);  // [3 pairs, I]
   A.act = act;
   A.queue = c->d_queue;
   if (ev) HIP_OK(c, hipEventRecord(ev[1], c->stream));
@@ -1011,8 +1027,9 @@ int moe_forward_dev(rbt_ctx *c, uint32_t layer, const float *x, size_t s, float 
   RBT_TRY(scratch_t(c, SC_TW, (size_t)P, &tw));
   size_t hi = std::max((size_t)I, L.shared_inter);
   // 2 * hi floats per pair: fp32 h for the GEMV path, or three bf16 parts (1.5 * I) for the MFMA path
-  RBT_TRY(scratch_t(c, SC_H, pslots * hi * 2, &h));
-  RBT_TRY(scratch_t(c, SC_YY, (size_t)npairs * H, &yy));
+  const size_t ybytes = align256((size_t)npairs * H * 4), area = ybytes + align256(pslots * hi * 8);
+  RBT_TRY(scratch_t(c, SC_YY, area / 4, &yy));
+  h = yy + ybytes / 4;
   int *dflags = c->d_flags;
 
   // profiling events: [0] start, [1] routing done, [2, 3] gate/up kernel, [4, 5] down kernel,
@@ -1119,10 +1136,10 @@ int moe_forward_dev(rbt_ctx *c, uint32_t layer, const float *x, size_t s, float 
   const bool grouped = !dgrouped && !mfma && S > 1 && (merge || !D.has_shared) &&
                        rbt::prefill_ok(L.routed_kind, H, I, (size_t)E, (size_t)k);
   const bool x3 = !dgrouped && !grouped && !mfma && (merge || !D.has_shared) &&
-                  x3_experts_ok(c, L.routed_kind, L.routed_gs, L.al16, x, S, k, E, H, I, D.has_shared ? 1 : 0);
+                  x3_experts_ok(c, L.routed_kind, L.routed_gs, L.al16, x, S, k, E, H, I, D.has_shared ? 1 : 0, area);
   if (x3) {
     RBT_TRY(x3_experts(c, L.routed_kind, L.d_table, L.d_shared, D.has_shared ? 1 : 0, x, S, k, E, H, I, ids, wts, ptok,
-                       tpair, tw, h, yy, RbtAct{}, c->prof ? ev.data() : nullptr));
+                       tpair, tw, yy, area, RbtAct{}, c->prof ? ev.data() : nullptr));
     HIP_OK(c, rbt::launch_combine(*c, yy, S, k, H, tpair, tw, shs, D.has_shared, gated, dst));
   } else if (dgrouped) {
     RBT_TRY(decode_grouped_dev(c, L, x, S, k, E, H, I, ids, wts, shs, ptok, tpair, tw, h, yy, gated, dst,
@@ -1357,8 +1374,10 @@ static int latent_moe_dev(rbt_ctx *c, uint32_t layer, const rbt_latent_moe_desc 
   RBT_TRY(scratch_t(c, SC_TPAIR, (size_t)P, &tpair));
   RBT_TRY(scratch_t(c, SC_TW, (size_t)P, &tw));
   RBT_TRY(scratch_t(c, SC_XL, (size_t)S * MH, &xl));
-  RBT_TRY(scratch_t(c, SC_H, pslots * I * 2, &h));
-  RBT_TRY(scratch_t(c, SC_YY, (size_t)P * MH, &yy));
+  // the pairs' rows, then h: 2 I floats per pair
+  const size_t ybytes = align256((size_t)P * MH * 4), area = ybytes + align256(pslots * I * 8);
+  RBT_TRY(scratch_t(c, SC_YY, area / 4, &yy));
+  h = yy + ybytes / 4;
   RBT_TRY(scratch_t(c, SC_ROUTED, (size_t)S * MH, &routed));
   int *dflags = c->d_flags;
   // routing of the full-width x (certified logits, exact folds where the order is not certain)
@@ -1426,9 +1445,9 @@ static int latent_moe_dev(rbt_ctx *c, uint32_t layer, const rbt_latent_moe_desc 
                                 nullptr, nullptr, yy, (size_t)P * MH));
     RBT_TRY(matmul_dev(c, xl, x, &lw->down_proj, s));
   }
-  if (x3_experts_ok(c, kind, gs, Ly.lat_al16, xl, S, K, (int)E, (int)MH, (int)I, 0)) {
-    RBT_TRY(x3_experts(c, kind, table, table + E, 0, xl, S, K, (int)E, (int)MH, (int)I, ids, wts, ptok, tpair, tw, h,
-                       yy, act, nullptr));
+  if (x3_experts_ok(c, kind, gs, Ly.lat_al16, xl, S, K, (int)E, (int)MH, (int)I, 0, area)) {
+    RBT_TRY(x3_experts(c, kind, table, table + E, 0, xl, S, K, (int)E, (int)MH, (int)I, ids, wts, ptok, tpair, tw, yy,
+                       area, act, nullptr));
   } else {
     if (!grp_in_select)
       HIP_OK(c, rbt::launch_group(*c, ids, wts, S, K, (int)E, table, table + E, pjob, ptok, tpair, tw,

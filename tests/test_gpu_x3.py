@@ -254,3 +254,21 @@ def test_router_of_short_prompts(own_ctx, H, E, S, cores):
     for t in range(0, S, 8):
         own_ctx.moe_forward(0, x[t:t + 1].contiguous(), 1, out, one)
         assert bool((ids[t] == one[0]).all()), t
+
+
+@pytest.mark.parametrize("E,k,shared,I,S", [(16, 1, False, 1024, 40), (16, 1, True, 512, 40), (4, 4, False, 512, 3)])
+def test_int4_layer_work_area(own_ctx, E, k, shared, I, S):
+    """One expert per token, with and without a shared one: what the tiled products keep beside the rows lies
+    between the rows and h, and a layer that leaves too little room there takes the GEMVs."""
+    import torch
+    H = 1024
+    m, _ = _device_layer(own_ctx, "i4g", H, I, E, k, shared, 700)
+    x, out = torch.from_numpy(normal((S, H), 5)).cuda(), torch.full((S + 1, H), 7.0, device="cuda")
+    ids, w = torch.empty(S, k, dtype=torch.int32, device="cuda"), torch.empty(S, k, device="cuda")
+    own_ctx.moe_forward(0, x, S, out[:S], ids, w)
+    want = _ffn64(own_ctx, m, E, x.double()) if shared else torch.zeros(S, H, dtype=torch.float64, device="cuda")
+    for e in range(E):
+        t, j = torch.nonzero(ids == e, as_tuple=True)
+        want[t] += w[t, j].double()[:, None] * _ffn64(own_ctx, m, e, x[t].double())
+    assert float(((out[:S].double() - want).norm(dim=1) / want.norm(dim=1)).max()) < 2e-6
+    assert bool((out[S] == 7.0).all())

@@ -65,9 +65,11 @@ def test_noalloc_small_layers(ctx, orc):
 
 
 # the last token counts whose buffers fit the fixed array
-@pytest.mark.parametrize("name,counts", [("c1", (26, 27, 28, 29)), ("c3", (35, 36, 37))])
+@pytest.mark.parametrize("name,counts", [("c1", (26, 27, 28, 29)), ("c2", (8, 24, 37, 38, 39, 40, 41)),
+                                         ("c3", (35, 36, 37))])
 def test_noalloc_short_prompts(own_ctx, name, counts):
-    """A prompt of 17 to 63 tokens: nothing the router may use is taken from what the experts need."""
+    """A prompt of 17 to 63 tokens: nothing the router may use is taken from what the experts need, and which
+    kernels run does not depend on the memory there is (c2: grouped int4 through the tiled products)."""
     import torch
     import rabbit_amd.workloads as W
     cfg = W.CONFIGS[name]
