@@ -939,7 +939,7 @@ constexpr long RB_LINE = 10000;
 // intervals for every (row, token) with a selection workgroup per token (whose idle waves write xb3_sel,
 // the tokens' three-part split, when given); larger batches on the matrix cores with a rigorous bound on
 // the distance to the reference's sequential fp32 fold, or as that fold itself. Below 64 tokens the
-// matrix-core logits' scratch is `spare` (spare_n floats: the layer's expert rows, written later), so that
+// matrix-core logits' scratch is `spare` (spare_n floats: the layer's expert rows and h, written later), so that
 // the choice depends on the shape alone and takes no memory the call's later buffers need; they run in as
 // many K parts as fit it (hidden 1536, 512 experts, top-4, 63 tokens: 176 us a call, 336 with certified logits).
 int route_logits_select(rbt_ctx *c, const rbt::RouterArgs &ra, int erows, const float *sgate, const RbtExpertDev *table,
@@ -1131,7 +1131,7 @@ int moe_forward_dev(rbt_ctx *c, uint32_t layer, const float *x, size_t s, float 
     if (dgrouped && !rbt::router_exact_ok(S, H) && rbt::router_batch_ok(ra) && al16({sgate, x}) && H % 4 == 0)
       RBT_TRY(scratch_t(c, SC_XB, (size_t)3 * S * H, &xb3_sel));
     RBT_TRY(route_logits_select(c, ra, erows, sgate, L.d_table, mid, bnd, ids, wts, shs, grp_in_select ? &ga : nullptr,
-                                sh_in_select ? &sgu : nullptr, xb3_sel, yy, (size_t)npairs * H));
+                                sh_in_select ? &sgu : nullptr, xb3_sel, yy, area / 4));
   }
   const bool grouped = !dgrouped && !mfma && S > 1 && (merge || !D.has_shared) &&
                        rbt::prefill_ok(L.routed_kind, H, I, (size_t)E, (size_t)k);
@@ -1442,7 +1442,7 @@ static int latent_moe_dev(rbt_ctx *c, uint32_t layer, const rbt_latent_moe_desc 
                                            (int)H, (int)MH, xl));
   } else {
     RBT_TRY(route_logits_select(c, ra, (int)E, nullptr, table, mid, bnd, ids, wts, shs, grp_in_select ? &ga : nullptr,
-                                nullptr, nullptr, yy, (size_t)P * MH));
+                                nullptr, nullptr, yy, area / 4));
     RBT_TRY(matmul_dev(c, xl, x, &lw->down_proj, s));
   }
   if (x3_experts_ok(c, kind, gs, Ly.lat_al16, xl, S, K, (int)E, (int)MH, (int)I, 0, area)) {
