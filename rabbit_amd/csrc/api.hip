@@ -858,18 +858,37 @@ X3Area x3_area(int S, int k, int E, int H, int I, int has_shared, size_t area) {
   return a;
 }
 
-bool x3_experts_ok(rbt_ctx *c, int kind, size_t gs, bool aligned, const float *x, int S, int k, int E, int H, int I,
-                   int has_shared, size_t area) {
-  // The tiled products stream each unique expert once, the GEMVs once per (token, expert) pair and
-  // somewhat faster. int4, hidden 6144, top-8 of 256 and a shared expert, us, GEMV against tiled: 4 tokens
-  // 197 / 203, 6 271 / 289, 8 345 / 333, 16 650 / 572, 40 1553 / 952: the line lies where the pairs are
-  // 1.22 times the experts that uniform routing picks. MXFP4 (moe_hidden 3584 x 3072, top-16 of 896):
-  // 4 tokens 320 / 336, 8 552 / 514, 16 970 / 834, 131 6.9 ms / 2.5 ms: 1.06 times.
+// Whether a batch's experts take the tiled products, which stream each unique expert once but leave the
+// CUs waiting where there are few tiles (a tile's rows run over all columns), rather than the GEMVs, which
+// stream an expert once per (token, expert) pair. In bytes: pairs x expert >= c x uniq x expert + a start-up
+// that grows with the columns of the two products; uniq is what uniform routing picks. us, GEMV against tiled,
+// int4 unless said (hidden x inter, experts, top-k, s: a shared one):
+//   6144 x 2048, 256, 8, s    6 tokens 261 / 283, 12 520 / 483, 24 939 / 689
+//   5120 x 1536, 160, 6, s    4 tokens 125 / 128,  6 165 / 150, 16 420 / 296
+//   4096 x 1536, 128, 8       8 tokens 184 / 207, 12 234 / 220, 24 440 / 304
+//   4096 x 1024,  16, 1, s    8 tokens  46 /  70, 16  65 /  72, 24  89 /  75
+//   2048 x 1024,  64, 6, s    8 tokens  76 /  82, 10  90 /  86, 24 172 / 103
+//   1024 x 512,   24, 4, s    4 tokens  36 /  38, 10  48 /  41, 24  72 /  45
+//   3584 x 3072, 896, 16      MXFP4 (latent): 6 tokens 376 / 380, 10 611 / 568, 24 1299 / 1101
+//   4096 x 3072,  32, 2       MXFP4 (latent): 10 tokens 128 / 142, 14 156 / 143, 24 224 / 164
+// Past 6144 columns the gate/up GEMV takes two column parts and its activation a launch of its own (7168 x
+// 2048, 256, 8, s: 4 tokens 247 / 235, 8 459 / 388); past 8192 the GEMVs read a row per workgroup (4096 x
+// 14336, 8, 2: 2 tokens 1390 / 177).
+bool x3_experts_win(int kind, size_t gs, int S, int k, int E, int H, int I, int has_shared) {
+  if (!rbt::decode_shape_ok(H, kind, gs) || !rbt::decode_shape_ok(I, kind, gs)) return true;
+  const bool i4 = kind == RBT_QT_I4_GROUPED;
+  const double expert = 3.0 * H * I * (i4 ? 0.625 : 0.53125);  // bytes
   const double uniq = E * (1.0 - std::pow(1.0 - std::min(1.0, (double)k / E), S)) + has_shared;
-  return S >= 2 && (double)S * (k + has_shared) >= (kind == RBT_QT_I4_GROUPED ? 1.22 : 1.06) * uniq && aligned &&
-         al16({x}) && (size_t)6 * S * H < ((size_t)1 << 32) && rbt::x3_ok(kind, gs, H, I, true) &&
+  const double per = H > 6144 ? 1.02 : i4 ? 1.2 : 1.04;
+  return S * (double)(k + has_shared) * expert >=
+         per * uniq * expert + std::min(100e6, (i4 ? 20e3 : 15e3) * ((double)H + I));
+}
+
+bool x3_experts_ok(int kind, size_t gs, bool aligned, const float *x, int S, int k, int E, int H, int I,
+                   int has_shared, size_t area) {
+  return S >= 2 && aligned && al16({x}) && (size_t)6 * S * H < ((size_t)1 << 32) && rbt::x3_ok(kind, gs, H, I, true) &&
          rbt::x3_ok(kind, gs, I, H, false) && E + 1 <= rbt::PG_MAXE &&
-         x3_area(S, k, E, H, I, has_shared, area).fits;
+         x3_experts_win(kind, gs, S, k, E, H, I, has_shared) && x3_area(S, k, E, H, I, has_shared, area).fits;
 }
 
 // A batch through its routed (and shared) experts with fp32 accuracy, every unique expert's weights
@@ -1136,7 +1155,7 @@ int moe_forward_dev(rbt_ctx *c, uint32_t layer, const float *x, size_t s, float 
   const bool grouped = !dgrouped && !mfma && S > 1 && (merge || !D.has_shared) &&
                        rbt::prefill_ok(L.routed_kind, H, I, (size_t)E, (size_t)k);
   const bool x3 = !dgrouped && !grouped && !mfma && (merge || !D.has_shared) &&
-                  x3_experts_ok(c, L.routed_kind, L.routed_gs, L.al16, x, S, k, E, H, I, D.has_shared ? 1 : 0, area);
+                  x3_experts_ok(L.routed_kind, L.routed_gs, L.al16, x, S, k, E, H, I, D.has_shared ? 1 : 0, area);
   if (x3) {
     RBT_TRY(x3_experts(c, L.routed_kind, L.d_table, L.d_shared, D.has_shared ? 1 : 0, x, S, k, E, H, I, ids, wts, ptok,
                        tpair, tw, yy, area, RbtAct{}, c->prof ? ev.data() : nullptr));
@@ -1445,7 +1464,7 @@ static int latent_moe_dev(rbt_ctx *c, uint32_t layer, const rbt_latent_moe_desc 
                                 nullptr, nullptr, yy, area / 4));
     RBT_TRY(matmul_dev(c, xl, x, &lw->down_proj, s));
   }
-  if (x3_experts_ok(c, kind, gs, Ly.lat_al16, xl, S, K, (int)E, (int)MH, (int)I, 0, area)) {
+  if (x3_experts_ok(kind, gs, Ly.lat_al16, xl, S, K, (int)E, (int)MH, (int)I, 0, area)) {
     RBT_TRY(x3_experts(c, kind, table, table + E, 0, xl, S, K, (int)E, (int)MH, (int)I, ids, wts, ptok, tpair, tw, yy,
                        area, act, nullptr));
   } else {

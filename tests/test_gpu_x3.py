@@ -89,7 +89,7 @@ def test_captured_batches(rbt_lib, orc):
 
 
 # 600 experts: the batch selection past 512; 24 experts of 3 to 40 tokens: every tile form with Situ
-@pytest.mark.parametrize("E,k,S", [(600, 4, 2), (600, 4, 40), (24, 4, 11), (24, 4, 60), (6, 4, 66)])
+@pytest.mark.parametrize("E,k,S", [(600, 4, 2), (600, 4, 40), (24, 4, 11), (24, 4, 16), (24, 4, 60), (6, 4, 66)])
 def test_latent_batches(ctx, orc, E, k, S):
     import rabbit_amd as R
     from test_gpu_latent import _latent_case, _run_latent
@@ -256,7 +256,8 @@ def test_router_of_short_prompts(own_ctx, H, E, S, cores):
         assert bool((ids[t] == one[0]).all()), t
 
 
-@pytest.mark.parametrize("E,k,shared,I,S", [(16, 1, False, 1024, 40), (16, 1, True, 512, 40), (4, 4, False, 512, 3)])
+@pytest.mark.parametrize("E,k,shared,I,S", [(16, 1, False, 1024, 40), (16, 1, True, 512, 40), (4, 4, False, 512, 3),
+                                               (4, 4, False, 8704, 3), (6, 6, True, 8704, 2)])
 def test_int4_layer_work_area(own_ctx, E, k, shared, I, S):
     """One expert per token, with and without a shared one: what the tiled products keep beside the rows lies
     between the rows and h, and a layer that leaves too little room there takes the GEMVs."""
@@ -272,3 +273,19 @@ def test_int4_layer_work_area(own_ctx, E, k, shared, I, S):
         want[t] += w[t, j].double()[:, None] * _ffn64(own_ctx, m, e, x[t].double())
     assert float(((out[:S].double() - want).norm(dim=1) / want.norm(dim=1)).max()) < 2e-6
     assert bool((out[S] == 7.0).all())
+
+
+@pytest.mark.parametrize("H,I,E,k,shared,S,tiled", [(4096, 1024, 16, 1, True, 8, False), (4096, 1024, 16, 1, True, 24, True),
+                                                    (1024, 1024, 8, 2, False, 6, False), (1024, 1024, 8, 2, False, 24, True),
+                                                    (512, 8704, 4, 1, False, 2, True)])
+def test_int4_layer_choice(own_ctx, H, I, E, k, shared, S, tiled):
+    """Where the tiles are too few to fill the chip the GEMVs run (the tiled products were up to 1.8 times as
+    long there)."""
+    import torch
+    _device_layer(own_ctx, "i4g", H, I, E, k, shared, 800)
+    x, out = torch.from_numpy(normal((S, H), 3)).cuda(), torch.empty(S, H, device="cuda")
+    own_ctx.profile_kernels()
+    own_ctx.moe_forward(0, x, S, out)
+    names = " ".join(own_ctx.profile_kernels_read())
+    own_ctx.profile_kernels(False)
+    assert ("k_x3I" in names) == tiled, names
