@@ -158,14 +158,14 @@ def _device_matrix(fmt, n, rows, cols, seed):
     return lambda e: R.QT.i4g(data[e], scale[e], rows, cols, 32)
 
 
-def _device_layer(ctx, fmt, H, I, E, k, shared, seed, layer=0, std=0.05, family=1, gated=False):
-    """A layer of device-resident experts: {"gate"/"up"/"down": e -> QT (E: the shared expert), "router"}."""
+def _device_layer(ctx, fmt, H, I, E, k, shared, seed, layer=0, std=0.05, family=1, gated=False, skip=()):
+    """A layer of device-resident experts (but for `skip`): {"gate"/"up"/"down": e -> QT (E: the shared expert), "router"}."""
     import torch
     import rabbit_amd as R
     m = {n: _device_matrix(fmt, E + 1, r, c, seed + i)
          for i, (n, r, c) in enumerate((("gate", I, H), ("up", I, H), ("down", H, I)))}
     slot = lambda e, eid: R.Slot(eid, m["down"](e), gate=m["gate"](e), up=m["up"](e))  # noqa: E731
-    for e in range(E):
+    for e in set(range(E)) - set(skip):
         ctx.pool_put(layer, slot(e, e))
     router = torch.from_numpy(normal((E, H), seed + 9, std)).cuda()
     gate = torch.from_numpy(normal(H, seed + 8, std)).cuda() if gated else None
@@ -289,3 +289,26 @@ def test_int4_layer_choice(own_ctx, H, I, E, k, shared, S, tiled):
     names = " ".join(own_ctx.profile_kernels_read())
     own_ctx.profile_kernels(False)
     assert ("k_x3I" in names) == tiled, names
+
+
+def test_missing_expert_of_a_batch(own_ctx):
+    """A picked expert without weights is an error, and the other experts' rows are what they are: its own count
+    as zeros, whatever the work area held."""
+    import torch
+    import rabbit_amd as R
+    H, I, E, k, S, gone = 1024, 1024, 8, 2, 40, 3
+    m, _ = _device_layer(own_ctx, "i4g", H, I, E, k, True, 900)
+    x, out = torch.from_numpy(normal((S, H), 5)).cuda(), torch.empty(S, H, device="cuda")
+    ids, w = torch.empty(S, k, dtype=torch.int32, device="cuda"), torch.empty(S, k, device="cuda")
+    own_ctx.moe_forward(0, x, S, out, ids, w)  # every expert there: leaves its rows behind
+    keep, _ = _device_layer(own_ctx, "i4g", H, I, E, k, True, 900, layer=1, skip=(gone,))
+    with pytest.raises(R.RbtError) as ei:
+        own_ctx.moe_forward(1, x, S, out, ids, w)
+    assert ei.value.status == R.abi.RBT_E_NOT_RESIDENT
+    assert bool((ids == gone).any())
+    want = _ffn64(own_ctx, m, E, x.double())
+    for e in range(E):
+        if e != gone:
+            t, j = torch.nonzero(ids == e, as_tuple=True)
+            want[t] += w[t, j].double()[:, None] * _ffn64(own_ctx, m, e, x[t].double())
+    assert float(((out.double() - want).norm(dim=1) / want.norm(dim=1)).max()) < 2e-6
