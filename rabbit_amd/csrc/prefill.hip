@@ -76,14 +76,19 @@ __device__ __forceinline__ uint32_t pg_load(const uint32_t *p) {
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
+// PSeg::rank: the rank, and whether the expert has no weights.
+constexpr int PG_RANK = 0xffff;
+__device__ __forceinline__ int pg_rank(int rank, int gone) { return (rank & PG_RANK) | gone << 16; }
+
 // Pair of pick p = t k + j. The slot of (t, e) within e's segment is the number of earlier tokens that
 // picked e. Token t's picks are written in pair order, which is unique_experts order (segments are in
 // rank order): pick j goes to position #{j' : key(j') < key(j)}, with key = rank of the expert, and
-// missing picks after every real one in slot order.
-template <typename RANK, typename OFF>
+// missing picks after every real one in slot order. A pick whose expert has no weights (gone) keeps its place
+// but names no pair: nothing writes that pair's row, and the combine leaves it out.
+template <typename RANK, typename OFF, typename GONE>
 __device__ __forceinline__ void pg_pair(int p, const int32_t *__restrict__ ids, const float *__restrict__ wts, int k,
-                                        int E, int W, int P, int has_shared, RANK rank, OFF off, const uint32_t *bits,
-                                        const uint32_t *pc, int *__restrict__ pair_tok, int *__restrict__ tok_pair,
+                                        int E, int W, int P, int has_shared, RANK rank, OFF off, GONE gone,
+                                        const uint32_t *bits, const uint32_t *pc, int *__restrict__ pair_tok, int *__restrict__ tok_pair,
                                         float *__restrict__ tok_w) {
   const int t = p / k, j = p - t * k;
   const int32_t *ti = ids + (long)t * k;
@@ -100,6 +105,7 @@ __device__ __forceinline__ void pg_pair(int p, const int32_t *__restrict__ ids, 
     const long wi = (long)e * W + (t >> 5);
     pr = off(e) + (int)(pc[wi] + __popc(bits[wi] & ((1u << (t & 31)) - 1u)));
     pair_tok[pr] = t;
+    if (gone(e)) pr = -1;
   }
   tok_pair[(long)t * k + pos] = pr;
   tok_w[(long)t * k + pos] = v ? wts[(long)t * k + j] : 0.0f;
@@ -128,6 +134,7 @@ __global__ __launch_bounds__(1024) void k_pgroup(const int32_t *__restrict__ ids
                                                  int *__restrict__ err, int *__restrict__ nuniq, int tch) {
   __shared__ int first[PG_MAXE], cnt[PG_MAXE], rank[PG_MAXE], byrank[PG_MAXE], segoff[PG_MAXE + 1];
   __shared__ uint32_t lbits[SMALL ? PG_SMALLW : 1], lpc[SMALL ? PG_SMALLW : 1];
+  __shared__ uint32_t gone[PG_MAXE / 32 + 1];  // experts picked that have no weights
   __shared__ int ws[17];
   __shared__ int carry_s;
   uint32_t *bits = SMALL ? lbits : gbits, *pc = SMALL ? lpc : gpc;
@@ -139,6 +146,7 @@ __global__ __launch_bounds__(1024) void k_pgroup(const int32_t *__restrict__ ids
     first[e] = 0x7fffffff;
     cnt[e] = 0;
   }
+  if (tid <= PG_MAXE / 32) gone[tid] = 0u;
   for (long i = tid; i < (long)E * W; i += 1024) bits[i] = 0u;
   if (!SMALL) __threadfence();
   __syncthreads();
@@ -151,7 +159,10 @@ __global__ __launch_bounds__(1024) void k_pgroup(const int32_t *__restrict__ ids
       atomicMin(&first[e], p);
       atomicOr(&bits[(long)e * W + (t >> 5)], 1u << (t & 31));
       const RbtExpertDev J = table[e];
-      if (J.gd == nullptr || J.ud == nullptr || J.dd == nullptr) atomicOr(err, 1);
+      if (J.gd == nullptr || J.ud == nullptr || J.dd == nullptr) {
+        atomicOr(err, 1);
+        atomicOr(&gone[e >> 5], 1u << (e & 31));
+      }
     }
   }
   if (!SMALL) __threadfence();
@@ -179,6 +190,7 @@ __global__ __launch_bounds__(1024) void k_pgroup(const int32_t *__restrict__ ids
     __syncthreads();
   }
   const int U = carry_s;
+  auto is_gone = [&](int e) { return (int)(gone[e >> 5] >> (e & 31) & 1u); };
   // segment offsets in rank order (two ranks per thread)
   {
     const int u0 = 2 * tid, u1 = 2 * tid + 1;
@@ -200,16 +212,16 @@ __global__ __launch_bounds__(1024) void k_pgroup(const int32_t *__restrict__ ids
     int tot;
     const int ex = pg_block_scan(n0 + n1, ws, &tot);
     if (u0 < nseg) {
-      segs[u0] = PSeg{u0 < U ? byrank[u0] : -1, u0 < U ? segoff[u0] : P, seg_cnt(u0), !SMALL && u0 < E ? rank[u0] : 0};
+      segs[u0] = PSeg{u0 < U ? byrank[u0] : -1, u0 < U ? segoff[u0] : P, seg_cnt(u0), !SMALL && u0 < E ? pg_rank(rank[u0], is_gone(u0)) : 0};
       for (int c = 0; c < n0; c++) tiles[ex + c] = PTile{u0, c * tch};
     } else if (!SMALL && u0 < E) {
-      segs[u0].rank = rank[u0];
+      segs[u0].rank = pg_rank(rank[u0], is_gone(u0));
     }
     if (u1 < nseg) {
-      segs[u1] = PSeg{u1 < U ? byrank[u1] : -1, u1 < U ? segoff[u1] : P, seg_cnt(u1), !SMALL && u1 < E ? rank[u1] : 0};
+      segs[u1] = PSeg{u1 < U ? byrank[u1] : -1, u1 < U ? segoff[u1] : P, seg_cnt(u1), !SMALL && u1 < E ? pg_rank(rank[u1], is_gone(u1)) : 0};
       for (int c = 0; c < n1; c++) tiles[ex + n0 + c] = PTile{u1, c * tch};
     } else if (!SMALL && u1 < E) {
-      segs[u1].rank = rank[u1];
+      segs[u1].rank = pg_rank(rank[u1], is_gone(u1));
     }
     if (tid == 0) {
       *ntiles = tot;
@@ -236,7 +248,7 @@ __global__ __launch_bounds__(1024) void k_pgroup(const int32_t *__restrict__ ids
   __syncthreads();
   for (int p = tid; p < P; p += 1024)
     pg_pair(p, ids, wts, k, E, W, P, has_shared, [&](int e) { return rank[e]; }, [&](int e) { return segoff[rank[e]]; },
-            bits, pc, pair_tok, tok_pair, tok_w);
+            is_gone, bits, pc, pair_tok, tok_pair, tok_w);
 }
 
 // The pairs of a call whose bitmaps are in global memory, one thread per (token, pick) over the chip: on
@@ -248,8 +260,8 @@ __global__ __launch_bounds__(256) void k_ppairs(const int32_t *__restrict__ ids,
                                                 float *__restrict__ tok_w) {
   const int p = blockIdx.x * 256 + threadIdx.x;
   if (p >= S * k) return;
-  pg_pair(p, ids, wts, k, E, (S + 31) >> 5, S * k, has_shared, [&](int e) { return segs[e].rank; },
-          [&](int e) { return segs[segs[e].rank].off; }, bits, pc, pair_tok, tok_pair, tok_w);
+  pg_pair(p, ids, wts, k, E, (S + 31) >> 5, S * k, has_shared, [&](int e) { return segs[e].rank & PG_RANK; },
+          [&](int e) { return segs[segs[e].rank & PG_RANK].off; }, [&](int e) { return segs[e].rank > PG_RANK; }, bits, pc, pair_tok, tok_pair, tok_w);
 }
 
 // x (fp32) -> bf16, round to nearest even. vec: x and xb allow 16- and 8-byte accesses.

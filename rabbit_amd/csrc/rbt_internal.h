@@ -172,7 +172,7 @@ struct PSeg {
   int eid;  // expert id, -1 for the shared expert
   int off;  // first pair of the segment
   int cnt;  // tokens (pairs) in the segment
-  int rank;  // entry e: the segment of expert e, when it is used
+  int rank;  // entry e: the segment of expert e, when it is used (pg_rank)
 };
 struct PTile {
   int seg;  // segment index

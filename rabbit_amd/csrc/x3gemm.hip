@@ -307,12 +307,11 @@ __device__ __forceinline__ void x3_run(const uint8_t *src, const uint32_t (&so)[
   }
 }
 
-// The tile of index ti: its expert, first pair and token count (none: nothing to do).
+// The tile of index ti: its expert, first pair and token count (0: nothing to do).
 struct X3Tile {
   RbtExpertDev J;
   int pbase, M;
   int n;  // single: the rows there are
-  bool absent;  // no weights: the tile's rows are zeros
 };
 __device__ __forceinline__ int x3_rows(const X3Args &A) { return A.nrows_dev ? min(A.nrows, *A.nrows_dev) : A.nrows; }
 
@@ -324,10 +323,9 @@ __device__ __forceinline__ X3Tile x3_tile(const X3Args &A, int ti) {
     T.J = s.eid >= 0 ? A.table[s.eid] : *A.shared_dev;
     T.pbase = s.off + t.c0;
     T.M = min(A.tch, s.cnt - t.c0);
-    T.absent = T.J.gd == nullptr || T.J.ud == nullptr || T.J.dd == nullptr;  // reported by k_pgroup
+    if (T.J.gd == nullptr || T.J.ud == nullptr || T.J.dd == nullptr) T.M = 0;  // reported by k_pgroup
     T.n = 0;
   } else {
-    T.absent = false;
     T.n = x3_rows(A);
     T.J = A.single;
     T.pbase = ti * A.tch;
@@ -448,10 +446,6 @@ __global__ __launch_bounds__(256, TOP == X3_BIG ? 2 : 3) void k_x3(const X3Args 
     const int ti = ub / RB, rb0 = ub - ti * RB;
     const X3Tile T = x3_tile(A, ti);
     if (T.M <= 0) {
-    } else if (T.absent) {
-      if (!GATEUP)  // the call reports the missing expert; its rows count as zeros, as with the GEMVs
-        for (int j = threadIdx.x; j < 32 * T.M; j += 256)
-          *reinterpret_cast<xf4 *>(A.y + (long)(T.pbase + j / 32) * A.O + 128 * rb0 + 4 * (j % 32)) = xf4{0.f, 0.f, 0.f, 0.f};
     } else if (T.M <= 5)
       x3_unit<I4, GATEUP, X3_SMALL>(A, T, KS, ks, rb0, lds);
     else if (TOP == X3_MID || T.M <= 16)
