@@ -428,11 +428,23 @@ const PoolEntry *find_pool_slot(rbt_ctx *c, const rbt_expert_slot *s) {
 }
 
 // Whether a batch through one matrix takes the tiled matrix-core kernels (split, product, sum of the K
-// parts: about 14 us of launches) rather than the GEMV per token, whose time grows with s. us, GEMV
-// against tiled: int4 7168 x 3584 s = 2 19.3 / 16.7, 3 25.2 / 16.9, 16 63.6 / 20.5, 512 1615 / 135; MXFP4 3584 x 3072
-// s = 4 9.7 / 14.3, 16 18.7 / 14.2, 64 55.5 / 21.2; 2048 x 8192 s = 4 10.0 / 14.0, 16 24.4 / 13.8.
-bool x3_matmul_wins(int kind, size_t s, size_t i, size_t o) {
-  return s >= 2 && s * i * o >= (size_t)(kind == RBT_QT_I4_GROUPED ? 75 : 100) * 1000000;
+// parts: 8-15 us of launches and latency) rather than the GEMV per token, whose time grows with s. The line
+// lies where s * columns * rows repays that, later for a matrix of less than 8 M weights (it stays in an
+// XCD's L2 for the GEMV; less so up to 1024 columns, where a tile's chain is short), earlier for many rows (whole tiles fill the chip) and past 6144 columns, where the
+// GEMV is slower; past 8192 columns the GEMV reads a row per workgroup. us, GEMV against tiled:
+//   MXFP4 4096 x 4096   s = 6 12.5 / 12.6, 8 13.4 / 12.6, 16 21.6 / 13.1   2048 x 8192  s = 5 11.0 / 10.0
+//         3584 x 3072   s = 8 11.0 / 11.9, 10 13.0 / 11.8                  8192 x 2048  s = 3 16.4 / 12.2
+//         2048 x 2048   s = 24 11.0 / 12.4, 33 14.9 / 12.8                 1024 x 1024  s = 100 12.8 / 12.3
+//   int4  4096 x 4096   s = 4 11.0 / 12.6, 5 14.0 / 12.6                   3584 x 7168  s = 3 15.0 / 13.0
+//         2048 x 2048   s = 24 13.4 / 14.0, 33 18.2 / 14.3                 8192 x 2048  s = 2 14.3 / 14.6, 3 19.0 / 14.5
+//         4096 x 1024   s = 24 14.5 / 15.6, 33 19.0 / 15.7                 16384 x 512  s = 2 92.9 / 20.2
+bool x3_matmul_wins(int kind, size_t gs, size_t s, size_t i, size_t o) {
+  const bool i4 = kind == RBT_QT_I4_GROUPED;
+  const size_t line = i > 6144            ? 45
+                      : i * o >= 8000000  ? (i4 ? 75 : o >= 8192 ? 80 : 105)
+                      : i > 1024          ? (i4 ? 104 : 120)
+                                          : (i4 ? 90 : 104);
+  return s >= 2 && (s * i * o >= line * 1000000 || !rbt::decode_shape_ok(i, kind, gs));
 }
 
 // Rows per tile: 32 where the rows of one matrix (or an expert, on average) go past 16.
@@ -482,7 +494,7 @@ int matmul_dev(rbt_ctx *c, float *y, const float *x, const rbt_qt *w, size_t s) 
     HIP_OK(c, rbt::launch_xgemv1(*c, (const uint8_t *)w->data, (const uint8_t *)w->scale, x, (int)i, (int)o, y));
     return RBT_OK;
   }
-  if (x3_matmul_wins(w->kind, s, i, o) && 6 * s * i < ((size_t)1 << 32) && al16({x, y, w->data, w->scale}) && rbt::x3_ok(w->kind, w->group_size, i, o, false)) {
+  if (x3_matmul_wins(w->kind, w->group_size, s, i, o) && 6 * s * i < ((size_t)1 << 32) && al16({x, y, w->data, w->scale}) && rbt::x3_ok(w->kind, w->group_size, i, o, false)) {
     const int rc = x3_matmul(c, y, x, w, s);
     if (rc <= 0) return rc;
   }
@@ -1483,7 +1495,7 @@ static int latent_moe_dev(rbt_ctx *c, uint32_t layer, const rbt_latent_moe_desc 
     HIP_OK(c, rbt::launch_proj1(*c, U.kind, U.group_size, U.data, U.scale, routed, (int)MH, (int)H, out, lw->norm,
                                 lw->eps));
   } else if (lw->norm && U.kind != RBT_QT_F32 && rbt::decode_shape_ok(MH, U.kind, U.group_size) &&
-      !x3_matmul_wins(U.kind, s, MH, H) &&
+      !x3_matmul_wins(U.kind, U.group_size, s, MH, H) &&
       ((uintptr_t)U.data | (uintptr_t)lw->norm) % 16 == 0) {
     // the norm of each summed row inside the up projection's waves, which read the whole row
     RBT_TRY(check_qt(c, &U, "matmul"));

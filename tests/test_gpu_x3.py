@@ -24,10 +24,10 @@ def _matrix(ctx, orc, fmt, rows, cols, seed):
     return w, ctx.dequant_rows(w, 0, rows).reshape(rows, cols).double()
 
 
-# tokens * columns * rows past the line where the tiled products take over; (2048, 1152): the GEMV below it
+# tokens * columns * rows about the line where the tiled products take over, the GEMV below it
 @pytest.mark.parametrize("fmt", ["mxfp4", "i4g"])
 @pytest.mark.parametrize("cols,rows,tokens", [(7168, 3584, (2, 4, 5, 6, 16, 17, 33)), (512, 16512, (12, 32, 49)),
-                                              (2048, 1152, (21, 22, 43, 48, 130)), (4608, 640, (34, 64, 65))])
+                                              (2048, 1152, (21, 22, 43, 48, 52, 130)), (4608, 640, (34, 41, 64, 65))])
 def test_matmul_batches(ctx, orc, fmt, cols, rows, tokens):
     import torch
     w, dense = _matrix(ctx, orc, fmt, rows, cols, cols + rows)
@@ -288,7 +288,7 @@ def test_int4_layer_choice(own_ctx, H, I, E, k, shared, S, tiled):
     own_ctx.moe_forward(0, x, S, out)
     names = " ".join(own_ctx.profile_kernels_read())
     own_ctx.profile_kernels(False)
-    assert ("k_x3I" in names) == tiled, names
+    assert ("4k_x3I" in names) == tiled, names
 
 
 # grouped int4 in one grouping launch and (more bitmap words than its LDS holds) in two, MXFP4 as a decode batch
@@ -316,3 +316,20 @@ def test_missing_expert_of_a_batch(own_ctx, fmt, I, E, k, S, tol):
             t, j = torch.nonzero(ids == e, as_tuple=True)
             want[t] += w[t, j].double()[:, None] * _ffn64(own_ctx, m, e, x[t].double())
     assert float(((out.double() - want).norm(dim=1) / want.norm(dim=1)).max()) < tol
+
+
+@pytest.mark.parametrize("fmt,cols,rows,s,tiled", [
+    ("mxfp4", 2048, 2048, 24, False), ("mxfp4", 2048, 2048, 33, True), ("mxfp4", 4096, 4096, 6, False),
+    ("mxfp4", 4096, 4096, 7, True), ("mxfp4", 8192, 2048, 2, False), ("mxfp4", 8192, 2048, 3, True),
+    ("mxfp4", 16384, 128, 2, True), ("mxfp4", 2048, 8192, 5, True), ("i4g", 2048, 2048, 24, False),
+    ("i4g", 2048, 2048, 33, True), ("i4g", 3584, 7168, 2, False), ("i4g", 3584, 7168, 3, True)])
+def test_matmul_choice(own_ctx, fmt, cols, rows, s, tiled):
+    """Small products keep the GEMV (the tiled ones were up to a sixth slower near the line)."""
+    import torch
+    q = _device_matrix(fmt, 1, rows, cols, 5)(0)
+    x, y = torch.from_numpy(normal((s, cols), 3)).cuda(), torch.empty(s, rows, device="cuda")
+    own_ctx.profile_kernels()
+    own_ctx.matmul_qt(y, x, q, s)
+    names = " ".join(own_ctx.profile_kernels_read())
+    own_ctx.profile_kernels(False)
+    assert ("4k_x3I" in names) == tiled, names
