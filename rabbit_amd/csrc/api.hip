@@ -450,34 +450,45 @@ bool x3_matmul_wins(int kind, size_t gs, size_t s, size_t i, size_t o) {
 // Rows per tile: 32 where the rows of one matrix (or an expert, on average) go past 16.
 int x3_tch(size_t rows) { return rows > 16 ? 32 : 16; }
 
+// Tokens of a batch through one matrix that go through the kernels at once, of s: the activations' parts take
+// at most X3_XB bytes whatever s is (a call of 65,536 tokens of 8192 columns would keep 4 GB otherwise). The
+// weights stream once per 32 tokens either way.
+constexpr size_t X3_XB = (size_t)256 << 20;
+size_t x3_matmul_run(size_t s, size_t i) {
+  return std::min(s, std::max<size_t>(32, X3_XB / (6 * i) / 32 * 32));
+}
+
 // A batch through one matrix on the matrix cores (x3gemm.hip): the activations' exact parts, then the
 // products, K split where the row blocks alone would leave CUs idle. Returns 1 when the scratch it
 // needs cannot be had (the caller takes another path).
 int x3_matmul(rbt_ctx *c, float *y, const float *x, const rbt_qt *w, size_t s) {
-  const size_t i = w->cols, o = w->rows;
+  const size_t i = w->cols, o = w->rows, run = x3_matmul_run(s, i);
   // (a bound over every s up to this one, so that a smaller batch never grows it)
   const int rb = rbt::x3_row_blocks((int)o, false);
-  const size_t part = rbt::x3_part_rows(*c, s, rb) * o;
-  if (!scratch_avail(c, {{SC_XB, 6 * s * i}, {SC_XP, 4 * part}})) return 1;
+  const size_t part = rbt::x3_part_rows(*c, run, rb) * o;
+  if (!scratch_avail(c, {{SC_XB, 6 * run * i}, {SC_XP, 4 * part}})) return 1;
   __bf16 *xb3;
   float *xp;
-  RBT_TRY(scratch_t(c, SC_XB, 3 * s * i, &xb3));
+  RBT_TRY(scratch_t(c, SC_XB, 3 * run * i, &xb3));
   RBT_TRY(scratch_t(c, SC_XP, part, &xp));
-  rbt::X3Args A;
-  A.single.dd = (const uint8_t *)w->data;
-  A.single.ds = w->scale;
-  A.nrows = A.S = (int)s;
-  A.xb3 = xb3;
-  A.K = (int)i;
-  A.O = (int)o;
-  A.tch = x3_tch(s);
-  A.wgs = rbt::x3_wgs(*c, A.tch);
-  const int ks = rbt::x3_ks((long)s, A.tch, (int)i, rb, A.wgs);
-  A.part = ks > 1;
-  A.y = A.part ? xp : y;
-  HIP_OK(c, rbt::launch_x3split(*c, w->kind, x, s, i, xb3));
-  HIP_OK(c, rbt::launch_x3(*c, w->kind, false, A));
-  if (A.part) HIP_OK(c, rbt::launch_x3sum(*c, xp, s * o, ks, y));
+  for (size_t t = 0; t < s; t += run) {
+    const size_t n = std::min(run, s - t);
+    rbt::X3Args A;
+    A.single.dd = (const uint8_t *)w->data;
+    A.single.ds = w->scale;
+    A.nrows = A.S = (int)n;
+    A.xb3 = xb3;
+    A.K = (int)i;
+    A.O = (int)o;
+    A.tch = x3_tch(n);
+    A.wgs = rbt::x3_wgs(*c, A.tch);
+    const int ks = rbt::x3_ks((long)n, A.tch, (int)i, rb, A.wgs);
+    A.part = ks > 1;
+    A.y = A.part ? xp : y + t * o;
+    HIP_OK(c, rbt::launch_x3split(*c, w->kind, x + t * i, n, i, xb3));
+    HIP_OK(c, rbt::launch_x3(*c, w->kind, false, A));
+    if (A.part) HIP_OK(c, rbt::launch_x3sum(*c, xp, n * o, ks, y + t * o));
+  }
   return RBT_OK;
 }
 
@@ -494,7 +505,8 @@ int matmul_dev(rbt_ctx *c, float *y, const float *x, const rbt_qt *w, size_t s) 
     HIP_OK(c, rbt::launch_xgemv1(*c, (const uint8_t *)w->data, (const uint8_t *)w->scale, x, (int)i, (int)o, y));
     return RBT_OK;
   }
-  if (x3_matmul_wins(w->kind, w->group_size, s, i, o) && 6 * s * i < ((size_t)1 << 32) && al16({x, y, w->data, w->scale}) && rbt::x3_ok(w->kind, w->group_size, i, o, false)) {
+  if (x3_matmul_wins(w->kind, w->group_size, s, i, o) && al16({x, y, w->data, w->scale}) &&
+      rbt::x3_ok(w->kind, w->group_size, i, o, false)) {
     const int rc = x3_matmul(c, y, x, w, s);
     if (rc <= 0) return rc;
   }
@@ -1311,7 +1323,8 @@ int apply_single_dev(rbt_ctx *c, const rbt_expert_slot *slot, const int32_t *ids
       rbt::x3_ok(kind, gs, d, i, true) && rbt::x3_ok(kind, gs, i, d, false)) {
     // a batch: the tiled products over the tokens that picked the expert (their number on the device), K
     // split by what it leaves idle. Partial sums' bounds hold for every s up to this one.
-    const size_t pg = rbt::x3_part_rows(*c, s, rbg) * 2 * i, pd = rbt::x3_part_rows(*c, s, rbd) * d;
+    const size_t pg = std::max(s, rbt::x3_part_rows(*c, s, rbg)) * 2 * i;
+    const size_t pd = std::max(s, rbt::x3_part_rows(*c, s, rbd)) * d;
     if (scratch_avail(c, {{SC_XB, 6 * s * d}, {SC_H, 6 * s * i}, {SC_XP, 4 * std::max(pg, pd)}, {SC_PTOK, 4 * s},
                           {SC_TW, 4 * s}, {SC_FLAGS, 16}})) {
       __bf16 *xb3, *hb3;

@@ -1,6 +1,7 @@
 // rbt_internal.h -- host-side declarations shared by the library's translation units.
 #pragma once
 
+#include <algorithm>
 #include <hip/hip_ext.h>
 #include <hip/hip_runtime.h>
 #include <stddef.h>
@@ -245,9 +246,11 @@ __host__ __device__ inline int x3_ks(long n, int tch, int cols, int row_blocks, 
   const int most = cols / 512 < X3_KSMAX ? cols / 512 : X3_KSMAX;
   return ks < 1 ? 1 : ks > most ? most : (int)ks;
 }
-// Rows of partial sums (each `matrices` x O floats) that x3_ks can ask for, over every n up to the given one.
+// Rows of partial sums (each `matrices` x O floats) that more than one K part can ask for, over every n up to
+// the given one: parts x n <= 8 n, and <= wgs tch / row_blocks + n while that many rows leave workgroups idle.
 inline size_t x3_part_rows(const Ctx &c, size_t n, int row_blocks) {
-  return 64 * (size_t)c.num_cu / row_blocks + n + 256;
+  const size_t idle = (64 * (size_t)c.num_cu + 256) / row_blocks + 1;  // (16 x 3 or 32 x 2 workgroups per CU)
+  return std::min(X3_KSMAX * n, idle + std::min(n, idle));
 }
 // One expert's tokens, found beside the split (rbt_single_rows).
 struct X3Pick {

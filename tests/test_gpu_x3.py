@@ -333,3 +333,30 @@ def test_matmul_choice(own_ctx, fmt, cols, rows, s, tiled):
     names = " ".join(own_ctx.profile_kernels_read())
     own_ctx.profile_kernels(False)
     assert ("4k_x3I" in names) == tiled, names
+
+
+@pytest.mark.parametrize("fmt", ["mxfp4", "i4g"])
+def test_matmul_runs(own_ctx, fmt):
+    """A batch whose activations' parts go through in three runs of 672, 672 and 57 tokens."""
+    import torch
+    cols, rows, s = 65536, 128, 1401
+    q = _device_matrix(fmt, 1, rows, cols, 6)(0)
+    g = torch.Generator(device="cuda")
+    g.manual_seed(4)
+    x, y = torch.randn(s, cols, device="cuda", generator=g), torch.full((s + 1, rows), 7.0, device="cuda")
+    own_ctx.matmul_qt(y[:s], x, q, s)
+    want = x.double() @ own_ctx.dequant_rows(q, 0, rows).reshape(rows, cols).double().t()
+    assert float(((y[:s].double() - want).norm(dim=1) / want.norm(dim=1)).max()) < 2e-6
+    assert bool((y[s] == 7.0).all())
+
+
+def test_matmul_scratch_is_bounded(own_ctx):
+    """What a large batch through one matrix leaves in the context does not grow with its tokens."""
+    import torch
+    cols, rows, s = 8192, 2048, 16384
+    q = _device_matrix("mxfp4", 1, rows, cols, 7)(0)
+    x, y = torch.randn(s, cols, device="cuda"), torch.empty(s, rows, device="cuda")
+    torch.cuda.synchronize()
+    free = torch.cuda.mem_get_info()[0]
+    own_ctx.matmul_qt(y, x, q, s)
+    assert free - torch.cuda.mem_get_info()[0] < 400 << 20
