@@ -132,6 +132,12 @@ struct rbt_ctx : rbt::Ctx {
   std::string err;
   void *scratch[SC_N] = {};
   size_t scratch_cap[SC_N] = {};
+  // slots handed out while the stream was capturing: a graph holds their address, so growth keeps the
+  // old buffer until the context ends
+  bool in_graph[SC_N] = {};
+  std::vector<void *> retired;
+  int call_capturing = -1;  // within a CallScope: whether the stream is capturing, once asked
+  int call_depth = 0;
   // allocation-free calls: the device's fixed scratch array (its device address, or nullptr when the
   // lookup failed), carved per slot for one call
   uint8_t *noalloc = nullptr;
@@ -216,8 +222,28 @@ int fail(rbt_ctx *c, int code, const char *fmt, ...) {
 size_t div_ceil(size_t a, size_t b) { return (a + b - 1) / b; }
 size_t align256(size_t n) { return (n + 255) & ~(size_t)255; }
 
+// One call that asks for many slots: whether the stream is capturing cannot change within it, and asking
+// takes 50 ns.
+struct CallScope {
+  rbt_ctx *c;
+  explicit CallScope(rbt_ctx *ctx) : c(ctx) {
+    if (c->call_depth++ == 0) c->call_capturing = -1;
+  }
+  ~CallScope() { c->call_depth--; }
+};
+
+bool capturing(rbt_ctx *c) {
+  if (c->call_depth && c->call_capturing >= 0) return c->call_capturing != 0;
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  const bool known = hipStreamIsCapturing(c->stream, &cap) == hipSuccess;
+  if (!known) (void)hipGetLastError();
+  c->call_capturing = !known || cap != hipStreamCaptureStatusNone;
+  return c->call_capturing != 0;
+}
+
 // Grow-only device scratch. Growth synchronises the stream first, so in-flight work never sees a
-// freed buffer. Inside an allocation-free call (c->arena set) the slots are carved out of the
+// freed buffer, and keeps a buffer that a captured graph may use (each growth is by a quarter at least, so
+// those add up to a few times the last one at most). Inside an allocation-free call (c->arena set) the slots are carved out of the
 // device's fixed scratch array instead, a slot keeping its region for the rest of the call.
 int scratch(rbt_ctx *c, int slot, size_t bytes, void **out) {
   if (bytes == 0) bytes = 256;
@@ -240,7 +266,11 @@ int scratch(rbt_ctx *c, int slot, size_t bytes, void **out) {
   }
   if (c->scratch_cap[slot] < bytes) {
     HIP_OK(c, hipStreamSynchronize(c->stream));
-    if (c->scratch[slot]) HIP_OK(c, hipFree(c->scratch[slot]));
+    if (c->in_graph[slot])
+      c->retired.push_back(c->scratch[slot]);
+    else if (c->scratch[slot])
+      HIP_OK(c, hipFree(c->scratch[slot]));
+    c->in_graph[slot] = false;
     c->scratch[slot] = nullptr;
     c->scratch_cap[slot] = 0;
     size_t cap = align256(bytes + bytes / 4);
@@ -250,6 +280,7 @@ int scratch(rbt_ctx *c, int slot, size_t bytes, void **out) {
     }
     c->scratch_cap[slot] = cap;
   }
+  if (!c->in_graph[slot]) c->in_graph[slot] = capturing(c);
   *out = c->scratch[slot];
   return RBT_OK;
 }
@@ -262,25 +293,14 @@ int scratch_t(rbt_ctx *c, int slot, size_t count, T **out) {
   return RBT_OK;
 }
 
-// Whether the call can have these scratch sizes: they fit the fixed array of an allocation-free call,
-// or the slots are large enough or can grow now (a stream under capture allocates nothing). False
-// leaves the call as it was, for a path that needs less.
+// Whether the call can have these scratch sizes: the slots are large enough or can grow now (a stream under
+// capture allocates nothing, nor does an allocation-free call). False leaves the call as it was, for a path
+// that needs less.
 bool scratch_avail(rbt_ctx *c, std::initializer_list<std::pair<int, size_t>> need) {
-  if (c->arena) {
-    size_t sum = 0;
-    for (const auto &n : need) {
-      if (c->arena_sz[n.first] == 0) sum += align256(std::max<size_t>(n.second, 1));
-      else if (c->arena_sz[n.first] < n.second) return false;
-    }
-    return sum <= c->arena_cap - c->arena_used;
-  }
+  if (c->arena) return false;
   for (const auto &n : need) {
     if (c->scratch[n.first] && c->scratch_cap[n.first] >= n.second) continue;
-    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(c->stream, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) {
-      (void)hipGetLastError();
-      return false;
-    }
+    if (capturing(c)) return false;
     void *p;
     const std::string err = c->err;
     if (scratch(c, n.first, n.second, &p) != RBT_OK) {
@@ -1034,6 +1054,7 @@ int moe_forward_dev(rbt_ctx *c, uint32_t layer, const float *x, size_t s, float 
   if (s == 0) return RBT_OK;
   if (!x || !out) return fail(c, RBT_E_INVALID, "null x or out");
   if (s > 65536) return fail(c, RBT_E_UNSUPPORTED, "more than 65536 tokens per call");
+  const CallScope scope(c);
   RBT_TRY(refresh_table(c, layer, L));
   const rbt_moe_layer_desc &D = L.desc;
   const int S = (int)s, E = (int)D.n_experts, H = (int)D.hidden, I = (int)D.moe_inter;
@@ -1395,6 +1416,7 @@ static int latent_moe_dev(rbt_ctx *c, uint32_t layer, const rbt_latent_moe_desc 
   if (s > (size_t)INT32_MAX / std::max<size_t>(k, 1)) return fail(c, RBT_E_INVALID, "too many tokens");
   RbtAct act;
   RBT_TRY(to_act(c, &lw->act, &act));
+  const CallScope scope(c);
   const int S = (int)s, K = (int)k, P = S * K;
   // the layer's pool slots seen at (moe_hidden, moe_inter), plus a zero job for the shared slots
   RBT_TRY(refresh_latent(c, layer, Ly, MH));
@@ -1594,6 +1616,7 @@ void rbt_destroy(rbt_ctx *c) {
     if (kv.second.alloc) (void)hipFree(kv.second.alloc);
   for (int i = 0; i < SC_N; i++)
     if (c->scratch[i]) (void)hipFree(c->scratch[i]);
+  for (void *p : c->retired) (void)hipFree(p);
   if (c->d_flags) (void)hipFree(c->d_flags);
   for (auto &r : c->ev_rows)
     for (auto e : r) c->ev_free.push_back(e);

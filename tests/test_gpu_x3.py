@@ -360,3 +360,54 @@ def test_matmul_scratch_is_bounded(own_ctx):
     free = torch.cuda.mem_get_info()[0]
     own_ctx.matmul_qt(y, x, q, s)
     assert free - torch.cuda.mem_get_info()[0] < 400 << 20
+
+
+def test_captures_outlive_larger_calls(own_ctx):
+    """A captured batch through one matrix and a captured decode batch of a layer replay right after larger
+    eager calls made the context's scratch grow: the graphs' buffers stay. The memory a growth gives back is
+    written over before each replay."""
+    import ctypes as C
+    import torch
+    H, I, E, k, S = 1024, 1024, 8, 2, 12
+    m, _ = _device_layer(own_ctx, "mxfp4", H, I, E, k, False, 950)
+    q = _device_matrix("i4g", 1, 3584, 7168, 8)(0)
+    dense = own_ctx.dequant_rows(q, 0, 3584).reshape(3584, 7168).double()
+    x, y = torch.empty(9, 7168, device="cuda"), torch.empty(9, 3584, device="cuda")
+    xl, out = torch.empty(S, H, device="cuda"), torch.empty(S, H, device="cuda")
+    lib, qc = own_ctx.lib, q.c()
+    product = lambda: lib.rbt_matmul_qt_d(own_ctx.h, y.data_ptr(), x.data_ptr(), C.byref(qc), 9)  # noqa: E731
+    layer = lambda: lib.rbt_moe_forward_d(own_ctx.h, 0, xl.data_ptr(), S, out.data_ptr(), None, None)  # noqa: E731
+
+    def fill(seed):
+        x.copy_(torch.from_numpy(normal((9, 7168), seed)))
+        xl.copy_(torch.from_numpy(normal((S, H), seed + 1)))
+        torch.cuda.synchronize()
+
+    fill(1)
+    graphs = []
+    for call in (product, layer):
+        assert call() == 0  # eager first: the scratch is there
+        own_ctx.sync()
+        g = HipGraph(own_ctx.stream)
+        g.begin()
+        rc = call()
+        g.end()
+        assert rc == 0
+        graphs.append(g)
+    for i, s in enumerate((700, 1500, 3000)):
+        print("larger calls", s, flush=True)
+        own_ctx.matmul_qt(torch.empty(s, 3584, device="cuda"), torch.randn(s, 7168, device="cuda"), q, s)
+        own_ctx.moe_forward(0, torch.randn(s, H, device="cuda"), s, torch.empty(s, H, device="cuda"))
+        torch.full((64 << 20,), float("nan"), device="cuda")
+        fill(10 + i)
+        for g in graphs:
+            g.launch()
+        own_ctx.sync()
+        got, want = y.clone(), x.double() @ dense.t()
+        assert float((got.double() - want).norm() / want.norm()) < 1e-6
+        rows = out.clone()
+        assert layer() == 0
+        own_ctx.sync()
+        assert torch.equal(rows, out)
+    for g in graphs:
+        g.destroy()
