@@ -1315,11 +1315,19 @@ int to_act(rbt_ctx *c, const rbt_activation *a, RbtAct *out) {
   return RBT_OK;
 }
 
-// Tokens from which one expert's batch takes the tiled products (five launches, about 28 us) rather than
-// GEMVs per token that picked it. Half of the tokens picking, us, GEMV against tiled: MXFP4 8192 x 2048
-// 4 tokens 29.2 / 28.4, 8 37.1 / 29.4, 64 170 / 45, 256 633 / 76; int4 4 tokens 31.0 / 29.9, 8 41.4 / 30.5,
-// 256 780 / 86.
-bool x3_expert_wins(size_t s) { return s >= 5; }
+// Whether one expert's batch of s tokens takes the tiled products (five launches) rather than GEMVs per token
+// that picked it (four or five, their time growing with those tokens). How many picked it is known on the
+// device only, so the line weighs the most either form can lose: tokens times the expert's bytes of 100 MB and
+// more. us, GEMV against tiled, n tokens picking (with the token list in parallel in both):
+//   MXFP4 8192 x 2048, s = 8   n = 0 14 / 18, 1 21 / 23, 2 24 / 23, 4 31 / 23, 8 44 / 26; s = 256 n = 128 443 / 72
+//         4096 x 1536, s = 12  n = 1 16 / 21, 4 20 / 21, 6 25 / 23, 12 32 / 23
+//         2048 x 1024, s = 32  n = 1 19 / 20, 16 24 / 23, 32 31 / 23
+//   int4  6144 x 2048, s = 5   n = 0 16 / 18, 1 23 / 27, 2 27 / 27, 5 43 / 28
+//         2048 x 1024, s = 8   n = 1 19 / 22, 8 21 / 25 (GEMV); 512 x 512, s = 64 n = 64 20 / 29 (GEMV)
+bool x3_expert_wins(int kind, size_t gs, size_t s, size_t d, size_t i) {
+  if (!rbt::decode_shape_ok(d, kind, gs) || !rbt::decode_shape_ok(i, kind, gs)) return s >= 2;
+  return s >= 5 && 3.0 * s * d * i * (kind == RBT_QT_I4_GROUPED ? 0.625 : 0.53125) >= 100e6;
+}
 
 int apply_single_dev(rbt_ctx *c, const rbt_expert_slot *slot, const int32_t *ids, const float *w, size_t s, size_t k,
                      const float *x, size_t d, size_t i, const RbtAct &act, float *out) {
@@ -1340,7 +1348,7 @@ int apply_single_dev(rbt_ctx *c, const rbt_expert_slot *slot, const int32_t *ids
     return RBT_OK;
   }
   const int rbg = rbt::x3_row_blocks((int)i, true), rbd = rbt::x3_row_blocks((int)d, false);
-  if (x3_expert_wins(s) && 6 * s * std::max(d, i) < ((size_t)1 << 32) && al16({x, out}) && al16(v) &&
+  if (x3_expert_wins(kind, gs, s, d, i) && 6 * s * std::max(d, i) < ((size_t)1 << 32) && al16({x, out}) && al16(v) &&
       rbt::x3_ok(kind, gs, d, i, true) && rbt::x3_ok(kind, gs, i, d, false)) {
     // a batch: the tiled products over the tokens that picked the expert (their number on the device), K
     // split by what it leaves idle. Partial sums' bounds hold for every s up to this one.

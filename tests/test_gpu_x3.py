@@ -102,7 +102,7 @@ def test_latent_batches(ctx, orc, E, k, S):
 
 
 # nobody, one, 5, 6, 16, 17, 33 and 300 of the tokens pick the expert; K parts on both products
-@pytest.mark.parametrize("fmt,d,i", [("mxfp4", 8192, 2048), ("i4g", 512, 512)])
+@pytest.mark.parametrize("fmt,d,i", [("mxfp4", 8192, 2048), ("i4g", 512, 8704), ("i4g", 512, 512)])
 @pytest.mark.parametrize("s,picks", [(9, 0), (5, 1), (7, 5), (20, 6), (16, 16), (47, 17), (49, 33), (300, 300)])
 def test_expert_batches(ctx, orc, fmt, d, i, s, picks):
     import torch
@@ -411,3 +411,20 @@ def test_captures_outlive_larger_calls(own_ctx):
         assert torch.equal(rows, out)
     for g in graphs:
         g.destroy()
+
+
+@pytest.mark.parametrize("fmt,d,i,s,tiled", [("mxfp4", 8192, 2048, 5, True), ("mxfp4", 6144, 2048, 4, False),
+                                             ("i4g", 2048, 1024, 25, False), ("i4g", 2048, 1024, 26, True),
+                                             ("i4g", 512, 512, 200, False), ("i4g", 512, 8704, 2, True)])
+def test_expert_choice(own_ctx, fmt, d, i, s, tiled):
+    """Small experts keep the GEMVs for longer (the tiled products were up to a fifth slower there)."""
+    import torch
+    import rabbit_amd as R
+    g, u, dn = (_device_matrix(fmt, 1, r, c, 5)(0) for r, c in ((i, d), (i, d), (d, i)))
+    ids, w = torch.zeros(s, 2, dtype=torch.int32, device="cuda"), torch.ones(s, 2, device="cuda")
+    x, out = torch.from_numpy(normal((s, d), 3)).cuda(), torch.zeros(s, d, device="cuda")
+    own_ctx.profile_kernels()
+    own_ctx.apply_single_expert(R.Slot(0, dn, gate=g, up=u), ids, w, s, 2, x, d, i, out)
+    names = " ".join(own_ctx.profile_kernels_read())
+    own_ctx.profile_kernels(False)
+    assert ("4k_x3I" in names) == tiled, names
