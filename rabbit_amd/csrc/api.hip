@@ -478,19 +478,30 @@ size_t x3_matmul_run(size_t s, size_t i) {
   return std::min(s, std::max<size_t>(32, X3_XB / (6 * i) / 32 * 32));
 }
 
+size_t x3_matmul_part(rbt_ctx *c, size_t run, size_t o) {
+  // (a bound over every s up to this one, so that a smaller batch never grows it)
+  return rbt::x3_part_rows(*c, run, rbt::x3_row_blocks((int)o, false)) * o;
+}
+
+// Whether a batch takes x3_matmul: by size, shape and alignment, and where its scratch can be had.
+bool x3_matmul_takes(rbt_ctx *c, const float *y, const float *x, const rbt_qt *w, size_t s) {
+  const size_t i = w->cols, o = w->rows;
+  if (!x3_matmul_wins(w->kind, w->group_size, s, i, o) || !al16({x, y, w->data, w->scale}) ||
+      !rbt::x3_ok(w->kind, w->group_size, i, o, false))
+    return false;
+  const size_t run = x3_matmul_run(s, i);
+  return scratch_avail(c, {{SC_XB, 6 * run * i}, {SC_XP, 4 * x3_matmul_part(c, run, o)}});
+}
+
 // A batch through one matrix on the matrix cores (x3gemm.hip): the activations' exact parts, then the
-// products, K split where the row blocks alone would leave CUs idle. Returns 1 when the scratch it
-// needs cannot be had (the caller takes another path).
+// products, K split where the row blocks alone would leave CUs idle.
 int x3_matmul(rbt_ctx *c, float *y, const float *x, const rbt_qt *w, size_t s) {
   const size_t i = w->cols, o = w->rows, run = x3_matmul_run(s, i);
-  // (a bound over every s up to this one, so that a smaller batch never grows it)
   const int rb = rbt::x3_row_blocks((int)o, false);
-  const size_t part = rbt::x3_part_rows(*c, run, rb) * o;
-  if (!scratch_avail(c, {{SC_XB, 6 * run * i}, {SC_XP, 4 * part}})) return 1;
   __bf16 *xb3;
   float *xp;
   RBT_TRY(scratch_t(c, SC_XB, 3 * run * i, &xb3));
-  RBT_TRY(scratch_t(c, SC_XP, part, &xp));
+  RBT_TRY(scratch_t(c, SC_XP, x3_matmul_part(c, run, o), &xp));
   for (size_t t = 0; t < s; t += run) {
     const size_t n = std::min(run, s - t);
     rbt::X3Args A;
@@ -525,11 +536,7 @@ int matmul_dev(rbt_ctx *c, float *y, const float *x, const rbt_qt *w, size_t s) 
     HIP_OK(c, rbt::launch_xgemv1(*c, (const uint8_t *)w->data, (const uint8_t *)w->scale, x, (int)i, (int)o, y));
     return RBT_OK;
   }
-  if (x3_matmul_wins(w->kind, w->group_size, s, i, o) && al16({x, y, w->data, w->scale}) &&
-      rbt::x3_ok(w->kind, w->group_size, i, o, false)) {
-    const int rc = x3_matmul(c, y, x, w, s);
-    if (rc <= 0) return rc;
-  }
+  if (x3_matmul_takes(c, y, x, w, s)) return x3_matmul(c, y, x, w, s);
   if (w->kind != RBT_QT_F32 && aligned && rbt::decode_shape_ok(i, w->kind, w->group_size)) {
     RbtExpertDev one{};
     one.dd = (const uint8_t *)w->data;
@@ -1538,8 +1545,7 @@ static int latent_moe_dev(rbt_ctx *c, uint32_t layer, const rbt_latent_moe_desc 
     HIP_OK(c, rbt::launch_proj1(*c, U.kind, U.group_size, U.data, U.scale, routed, (int)MH, (int)H, out, lw->norm,
                                 lw->eps));
   } else if (lw->norm && U.kind != RBT_QT_F32 && rbt::decode_shape_ok(MH, U.kind, U.group_size) &&
-      !x3_matmul_wins(U.kind, U.group_size, s, MH, H) &&
-      ((uintptr_t)U.data | (uintptr_t)lw->norm) % 16 == 0) {
+             ((uintptr_t)U.data | (uintptr_t)lw->norm) % 16 == 0 && !x3_matmul_takes(c, out, routed, &U, s)) {
     // the norm of each summed row inside the up projection's waves, which read the whole row
     RBT_TRY(check_qt(c, &U, "matmul"));
     RbtExpertDev one{};

@@ -428,3 +428,18 @@ def test_expert_choice(own_ctx, fmt, d, i, s, tiled):
     names = " ".join(own_ctx.profile_kernels_read())
     own_ctx.profile_kernels(False)
     assert ("4k_x3I" in names) == tiled, names
+
+
+def test_latent_norm_in_the_projection(own_ctx, orc):
+    """An up projection that is large enough for the tiled product but of a shape it does not take keeps the norm
+    inside its GEMV (no launch of its own for the norm)."""
+    import rabbit_amd as R
+    from test_gpu_latent import _latent_case, _run_latent
+    H, MH, I, E, k, S = 1088, 1024, 64, 4, 2, 96
+    L, dq, uq, _ = _latent_case(own_ctx, orc, 0, H, MH, I, E, k, 7000, "i4g", 1.0)
+    norm = np.abs(normal(MH, 5, 1.0)) + np.float32(0.5)
+    own_ctx.profile_kernels()
+    _run_latent(own_ctx, R, 0, L, dq, uq, normal((S, H), 2), S, MH, norm, orc.situ(4.0, 25.0), R.situ(4.0, 25.0))
+    names = " ".join(own_ctx.profile_kernels_read())
+    own_ctx.profile_kernels(False)
+    assert "k_rmsnorm" not in names, names
