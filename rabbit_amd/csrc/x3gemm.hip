@@ -88,20 +88,29 @@ __device__ __forceinline__ xb8 x3_b(uint32_t w, float sc) {
 }
 
 // x = p[0] + p[1] + p[2] exactly: each part the leading 8 significant bits of what is left. An
-// infinite or NaN x keeps itself in p[0] and zeros in the others.
+// infinite or NaN x is all three parts. MXFP4 weights may be infinite (E8M0 253 and 254), and a part that is
+// zero would make NaN of a product that is infinite: from 2^-95 on such a part is 2^-126 with the sign of x,
+// which adds 2^-30 of the exact product at most and is rounded away from every sum that is not itself as small
+// (parts dealt out evenly stay exact but cost precision: bf16 activations 6.8e-8 -> 7.2e-8 from 64 bits).
+template <bool I4>
 __device__ __forceinline__ void x3_split(float x, __bf16 (&p)[3]) {
   const uint32_t b = __float_as_uint(x);
   if ((b & 0x7F800000u) == 0x7F800000u) {
-    p[0] = (__bf16)x;
-    p[1] = p[2] = (__bf16)0.0f;
+    p[0] = p[1] = p[2] = (__bf16)x;
     return;
   }
   const float h = __uint_as_float(b & 0xFFFF0000u);
   const float r = __fsub_rn(x, h);
-  const float m = __uint_as_float(__float_as_uint(r) & 0xFFFF0000u);
+  float m = __uint_as_float(__float_as_uint(r) & 0xFFFF0000u);
+  float l = __fsub_rn(r, m);
+  if (!I4 && (b & 0x7F800000u) >= (32u << 23)) {
+    const float tiny = __uint_as_float((b & 0x80000000u) | (1u << 23));
+    m = m == 0.0f ? tiny : m;
+    l = l == 0.0f ? tiny : l;
+  }
   p[0] = (__bf16)h;
   p[1] = (__bf16)m;
-  p[2] = (__bf16)__fsub_rn(r, m);
+  p[2] = (__bf16)l;
 }
 
 // 8 consecutive columns of one row: the parts (in x3_pos order), part_stride apart.
@@ -111,7 +120,7 @@ __device__ __forceinline__ void x3_write8(const float (&v)[8], __bf16 *__restric
 #pragma unroll
   for (int e = 0; e < 8; e++) {
     __bf16 p[3];
-    x3_split(v[e], p);
+    x3_split<I4>(v[e], p);
 #pragma unroll
     for (int q = 0; q < 3; q++) o[q][x3_pos(I4, e)] = p[q];
   }
@@ -388,7 +397,7 @@ __device__ __forceinline__ void x3_unit(const X3Args &A, const X3Tile &T, int KS
         A.y[((long)(ks * NM + t / TILES) * T.n + pr) * O + o0 + 16 * (t % TILES)] = v[t];
     } else if (GATEUP) {
       __bf16 p[3];
-      x3_split(rbt_act(A.act, v[0], v[NT - 1]), p);
+      x3_split<I4>(rbt_act(A.act, v[0], v[NT - 1]), p);
       __bf16 *d = A.hb3 + 3 * pr * O + (o0 & ~7) + x3_pos(I4, o0 & 7);
 #pragma unroll
       for (int q = 0; q < 3; q++) d[(long)q * O] = p[q];

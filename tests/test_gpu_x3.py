@@ -443,3 +443,60 @@ def test_latent_norm_in_the_projection(own_ctx, orc):
     names = " ".join(own_ctx.profile_kernels_read())
     own_ctx.profile_kernels(False)
     assert "k_rmsnorm" not in names, names
+
+
+@pytest.mark.parametrize("s", [9, 20, 36])
+def test_extreme_mxfp4_scales(own_ctx, s):
+    """Infinite and nearly infinite weights (E8M0 253 and 254; a block of 255 is NaN, as in the GEMVs), the smallest
+    scales, infinite and NaN activations: each output is the infinity, the NaN or the number that the 64-bit
+    product gives. Activations of 1 to 24
+    significant bits meet the infinite weights, so that their lower parts are zero or not. Tiles of up to 5, 16
+    and 32 tokens."""
+    import torch
+    import rabbit_amd as R
+    rows, cols = 3584, 3584
+    g = torch.Generator(device="cuda")
+    g.manual_seed(9)
+    data = torch.randint(0, 256, (rows, cols // 2), dtype=torch.uint8, device="cuda", generator=g)
+    scale = torch.randint(119, 124, (rows, cols // 32), dtype=torch.uint8, device="cuda", generator=g)
+    data[:8, 160:176] = 0                    # block 10 of the first rows: zeros but for one code
+    for row, byte, code in ((0, 254, 7), (1, 254, 15), (2, 254, 1), (3, 253, 7), (5, 0, 7), (6, 1, 1)):
+        scale[row, 10], data[row, 160] = byte, code
+    data[4, 160:176], scale[4, 10] = 0x77, 255
+    x = torch.randn(s, cols, device="cuda", generator=g)
+    x[:, 320:352] = torch.randn(s, 32, device="cuda", generator=g).abs().bfloat16().float().clamp(0.25, 1.9)
+    x[0, 320], x[1, 320], x[2, 320], x[3, 320], x[4, 320] = 1.0, -1.5, 1.0 + 2.0 ** -10, 1.0 + 2.0 ** -23, -0.75
+    x[5, 40], x[6, 40], x[7, 40] = float("inf"), -float("inf"), float("nan")
+    w = R.QT.mxfp4(data, scale, rows, cols)
+    y = torch.empty(s, rows, device="cuda")
+    own_ctx.matmul_qt(y, x, w, s)
+    dense = own_ctx.dequant_rows(w, 0, rows).reshape(rows, cols).double()
+    want = torch.stack([(x[t].double()[None, :] * dense).sum(1) for t in range(s)])
+    assert int(torch.isinf(want[:5, [0, 1, 3]]).sum()) == 15
+    want[:, 4] = float("nan")
+    fin = torch.isfinite(want)
+    assert bool((torch.isnan(want) == torch.isnan(y)).all())
+    inf = torch.isinf(want)
+    assert bool((want[inf] == y[inf].double()).all())
+    err = (y[fin].double() - want[fin]).abs() / want.abs().masked_fill(~fin, 0).amax(1, keepdim=True).expand_as(want)[fin]
+    assert float(err.max()) < 1e-5
+    ordinary = fin.clone()
+    ordinary[:, :8] = False
+    assert float((y.double() - want)[ordinary].norm() / want[ordinary].norm()) < 1e-6
+
+
+def test_precision_of_short_activations(own_ctx):
+    """Activations that are bf16 values: no further from 64 bits than full ones (the bar of test_matmul_batches)."""
+    import torch
+    q = _device_matrix("mxfp4", 1, 3584, 7168, 11)(0)
+    dense = own_ctx.dequant_rows(q, 0, 3584).reshape(3584, 7168).double()
+    for s in (4, 16, 64):
+        x = torch.from_numpy(normal((s, 7168), s)).cuda()
+        errs = []
+        for v in (x.bfloat16().float(), x):
+            y = torch.empty(s, 3584, device="cuda")
+            own_ctx.matmul_qt(y, v, q, s)
+            want = v.double() @ dense.t()
+            errs.append(float((y.double() - want).norm() / want.norm()))
+        print("error against 64 bits", s, errs)
+        assert errs[0] < 1e-6
