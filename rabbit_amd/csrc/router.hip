@@ -1308,8 +1308,9 @@ __device__ __forceinline__ void select3_body(SelLds &L, const SelParams &P, cons
     }
     __syncthreads();
   }
-  double gate_mid = P.erows > E ? ms[E] : 0.0;
+  [[maybe_unused]] double gate_mid = 0.0;  // REFINE: the shared gate's logit
   if constexpr (REFINE) {
+    if (P.erows > E) gate_mid = ms[E];
     for (int r = wave; r < kk; r += 4) {
       const float l = (float)logit_wave_f64(P.x + (size_t)s * P.H, P.W + (size_t)r_id[r] * P.H, P.H);
       if (lane == 0 && isfinite(l)) r_l[r] = l;  // (not finite: the fold's own value stays)
@@ -1329,7 +1330,7 @@ __device__ __forceinline__ void select3_body(SelLds &L, const SelParams &P, cons
       io[r] = r < kk ? r_id[r] : -1;
       wo[r] = r < kk ? s_w[r] : 0.0f;
     }
-    if (lane == 0 && sh_scale) sh_scale[s] = (P.erows > E) ? sigmoid_ref(__double2float_rn(gate_mid)) : 1.0f;
+    if (lane == 0 && sh_scale) sh_scale[s] = (P.erows > E) ? sigmoid_ref(__double2float_rn(REFINE ? gate_mid : ms[E])) : 1.0f;
     if (grp) {
       // single token: pair j = slot j; the shared expert is at G.shared_slot
       auto put = [&](int r, const uint8_t *gd, const void *gs, const uint8_t *ud, const void *us, const uint8_t *dd,
