@@ -88,12 +88,13 @@ def test_captured_batches(rbt_lib, orc):
     ctx.close()
 
 
-# 600 experts: the batch selection past 512; 24 experts of 3 to 40 tokens: every tile form with Situ
-@pytest.mark.parametrize("E,k,S", [(600, 4, 2), (600, 4, 40), (24, 4, 11), (24, 4, 16), (24, 4, 60), (6, 4, 66)])
+# 600 experts: the batch selection past 512 (the tiles from 80 tokens on); 24 experts of 1 to 40 tokens: every tile
+# form with Situ
+@pytest.mark.parametrize("E,k,S", [(600, 4, 2), (600, 4, 40), (600, 4, 80), (24, 4, 11), (24, 4, 16), (24, 4, 60), (6, 4, 66)])
 def test_latent_batches(ctx, orc, E, k, S):
     import rabbit_amd as R
     from test_gpu_latent import _latent_case, _run_latent
-    H, MH, I = 1024, 512, 512 if E < 600 else 64
+    H, MH, I = 1024, 512, 512 if E < 600 or S == 80 else 64
     layer = 70 + E % 7
     L, dq, uq, _ = _latent_case(ctx, orc, layer, H, MH, I, E, k, 4000 + E, "i4g", 1.0)
     x = normal((S, H), S, 1.0)
@@ -500,3 +501,82 @@ def test_precision_of_short_activations(own_ctx):
             errs.append(float((y.double() - want).norm() / want.norm()))
         print("error against 64 bits", s, errs)
         assert errs[0] < 1e-6
+
+
+@pytest.mark.parametrize("fmt", ["mxfp4", "i4g"])
+@pytest.mark.parametrize("what", ["x", "y", "data", "scale"])
+def test_matmul_unaligned(own_ctx, fmt, what):
+    """A batch whose x, y, codes or scales are not 16-byte aligned keeps the kernels that take them."""
+    import torch
+    import rabbit_amd as R
+    cols, rows, s = 2048, 2048, 40
+    q = _device_matrix(fmt, 1, rows, cols, 12)(0)
+
+    def off(t, skip):  # the tensor's values, its first byte `skip` bytes past a 16-byte boundary
+        n = skip // t.element_size()
+        b = torch.empty(t.numel() + 32, dtype=t.dtype, device="cuda")[n:n + t.numel()].view(t.shape)
+        b.copy_(t)
+        assert b.data_ptr() % 16 == skip
+        return b
+
+    x, y = torch.from_numpy(normal((s, cols), 3)).cuda(), torch.empty(s, rows, device="cuda")
+    data, scale = q.data, q.scale
+    want = x.double() @ own_ctx.dequant_rows(q, 0, rows).reshape(rows, cols).double().t()
+    x, y = (off(x, 4) if what == "x" else x), (off(y, 4) if what == "y" else y)
+    data, scale = (off(data, 8) if what == "data" else data), (off(scale, 4) if what == "scale" else scale)
+    w = R.QT.mxfp4(data, scale, rows, cols) if fmt == "mxfp4" else R.QT.i4g(data, scale, rows, cols, 32)
+    own_ctx.profile_kernels()
+    own_ctx.matmul_qt(y, x, w, s)
+    names = " ".join(own_ctx.profile_kernels_read())
+    own_ctx.profile_kernels(False)
+    assert "4k_x3I" not in names
+    assert float((y.double() - want).norm() / want.norm()) < 1e-6
+
+
+@pytest.mark.parametrize("latent", [False, True])
+def test_captured_layer_batches(own_ctx, orc, latent):
+    """An int4 layer's batch and a latent one, captured after an eager call: every replay is the eager call, bit for
+    bit, with eager calls in between."""
+    import ctypes as C
+    import torch
+    import rabbit_amd as R
+    from rabbit_amd import abi
+    from test_gpu_latent import _latent_case
+    lib, p = own_ctx.lib, lambda t: t.data_ptr()  # noqa: E731
+    k, S = 4, 60
+    if latent:
+        H, MH, E = 1024, 512, 24
+        _, dq, uq, _ = _latent_case(own_ctx, orc, 0, H, MH, 512, E, k, 8000, "i4g", 1.0)
+        keep = [torch.from_numpy(a).cuda() for q in (dq, uq) for a in (q.data, q.scale)]
+        norm = torch.ones(MH, device="cuda")
+        lw = abi.RbtLatentMoeDesc(MH, R.QT.i4g(keep[0], keep[1], MH, H, 32).c(), R.QT.i4g(keep[2], keep[3], H, MH, 32).c(),
+                                  p(norm), 1e-5, R.situ(4.0, 25.0))
+        call = lambda x, o, i, w: lib.rbt_latent_moe_d(own_ctx.h, 0, C.byref(lw), p(x), S, p(o), p(i), p(w))  # noqa: E731
+    else:
+        H, E = 1024, 24
+        _device_layer(own_ctx, "i4g", H, 1024, E, k, True, 1000)
+        call = lambda x, o, i, w: lib.rbt_moe_forward_d(own_ctx.h, 0, p(x), S, p(o), p(i), p(w))  # noqa: E731
+    new = lambda: [torch.empty(S, H, device="cuda"), torch.empty(S, k, dtype=torch.int32, device="cuda"),  # noqa: E731
+                   torch.empty(S, k, device="cuda")]
+    x, got, want = torch.from_numpy(normal((S, H), 1)).cuda(), new(), new()
+    torch.cuda.synchronize()
+    own_ctx.profile_kernels()
+    assert call(x, *got) == 0
+    own_ctx.sync()
+    assert "4k_x3I" in " ".join(own_ctx.profile_kernels_read())
+    own_ctx.profile_kernels(False)
+    g = HipGraph(own_ctx.stream)
+    g.begin()
+    rc = call(x, *got)
+    g.end()
+    assert rc == 0
+    for i in range(3):
+        x.copy_(torch.from_numpy(normal((S, H), 20 + i)))
+        torch.cuda.synchronize()
+        g.launch()
+        own_ctx.sync()
+        assert call(x, *want) == 0
+        own_ctx.sync()
+        for a, b in zip(got, want):
+            assert torch.equal(a, b)
+    g.destroy()
