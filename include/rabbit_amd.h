@@ -80,6 +80,11 @@ const char *rbt_last_error(const rbt_ctx *ctx);
 int rbt_sync(rbt_ctx *ctx);
 /* The context's hipStream_t, for callers that enqueue their own work around the `_d` calls. */
 void *rbt_stream(rbt_ctx *ctx);
+/* Graph capture: the asynchronous _d calls can be captured on this stream once a call of the same size
+ * has run eagerly, since scratch grows outside a capture only; layer calls then run the same kernels. A
+ * batch through one matrix can be captured without that: it then runs kernels that need no scratch, whose
+ * sums round differently. Scratch handed out under capture is kept until rbt_destroy, so a graph stays
+ * valid when later calls grow it. */
 /* Library version string. */
 const char *rbt_version(void);
 
@@ -259,7 +264,7 @@ int rbt_moe_forward_d(rbt_ctx *ctx, uint32_t layer, const float *x, size_t s, fl
  * per-call device buffer carved out of one fixed array of RBT_NOALLOC_SCRATCH_BYTES per device
  * (allocated when the library is loaded and held until the process ends), so the call itself
  * allocates nothing. Same kernels and results as rbt_moe_forward_d. A call whose buffers would not
- * fit returns RBT_E_UNSUPPORTED (e.g. the Qwen3.8-shaped layer fits up to 16 tokens, not a
+ * fit returns RBT_E_UNSUPPORTED (e.g. the Qwen3.8-shaped layer fits up to 29 tokens, not a
  * 512-token prefill). Every call on one device shares that device's array: calls that overlap on
  * one GPU (two contexts, two host threads) race. The layer must have been set (rbt_moe_layer_set*),
  * which sizes the layer's own tables. */

@@ -2,8 +2,10 @@
 // matrix cores: grouped gate/up and down over every expert of a call, one expert, or one matrix.
 //
 // The reference's s > 1 products (kernels.rs:233 matmul_mxfp4, :276 matmul_i4_grouped) read a weight
-// row once for all tokens. Here a workgroup takes a tile of up to X3_TCH = 32 tokens and a block of
-// rows, so a weight byte comes from HBM once per tile. Both operands are exact in bf16 parts:
+// row once for all tokens. Here a workgroup takes a tile of up to X3Args::tch tokens and a block of rows, so
+// a weight byte comes from HBM once per tile of its expert. tch is 16, or 32 where an expert has more than
+// 16 tokens on average (x3_tch; one expert's batch: from 49 tokens on); the shared expert of S tokens has
+// S / tch tiles. Both operands are exact in bf16 parts:
 //   activations  x = hi + mid + lo, three truncated bf16 parts (8 significant bits each: exact);
 //   MXFP4        e2m1 * 2^(b-127), exact in bf16 (v_cvt_scalef32_pk_bf16_fp4);
 //   grouped int4 the value -8..7 as sign and magnitude in an e4m3 byte (magnitudes 0..8 are m * 2^-9:
@@ -30,8 +32,8 @@
 // shared by the four waves. Three workgroups per CU for tiles of 16 tokens, two for 32.
 //
 // What bounds it, hidden 6144, 256 int4 experts of 2048, 301 tokens (283 tiles): gate/up 1.19 ms for
-// 4.5 GB of tiles (3.8 TB/s), against 7.77 ms for a GEMV per token and expert. VALU 50%, LDS 45% and
-// MFMA 23% busy, waves waiting a quarter of their cycles; without activation loads 1.03 ms, with a third
+// 4.5 GB of tiles (3.8 TB/s), against 7.77 ms for a GEMV per token and expert. VALU 61%, LDS 45% and
+// MFMA 27% busy, waves waiting a quarter of their cycles; without activation loads 1.03 ms, with a third
 // of the MFMAs 1.06. Tried: the MFMA layout loaded straight from memory (16 rows x 64 bytes) and
 // transposed by permlane swaps 2.16 ms; 512-column groups at two workgroups per CU 1.37; units in
 // contiguous runs over all XCDs 1.27 (6.6 GB fetched); static dealing 1.29; the stored code with the -8
@@ -487,7 +489,7 @@ __global__ __launch_bounds__(256) void k_x3sum(const xf4 *__restrict__ part, lon
 
 // Gate/up: h = act(sum of gate parts, sum of up parts), as the down product's activation parts. Four
 // threads per 8 columns of a row, each summing every fourth part (one thread summing them all waits for
-// memory once per part: 12.6 us at 16 parts); rows past *nrows_dev are left alone.
+// memory once per part, of which there are up to X3_KSMAX); rows past *nrows_dev are left alone.
 template <bool I4>
 __global__ __launch_bounds__(256) void k_x3act(const X3Args A) {
   const int o8 = A.O >> 3, q4 = threadIdx.x & 3;
