@@ -243,8 +243,9 @@ bool capturing(rbt_ctx *c) {
 
 // Grow-only device scratch. Growth synchronises the stream first, so in-flight work never sees a
 // freed buffer, and keeps a buffer that a captured graph may use (each growth is by a quarter at least, so
-// those add up to a few times the last one at most). Inside an allocation-free call (c->arena set) the slots are carved out of the
-// device's fixed scratch array instead, a slot keeping its region for the rest of the call.
+// those add up to a few times the last one at most). Inside an allocation-free call (c->arena set) the
+// slots are carved out of the device's fixed scratch array instead, a slot keeping its region for the rest
+// of the call.
 int scratch(rbt_ctx *c, int slot, size_t bytes, void **out) {
   if (bytes == 0) bytes = 256;
   if (c->arena) {
@@ -450,8 +451,9 @@ const PoolEntry *find_pool_slot(rbt_ctx *c, const rbt_expert_slot *s) {
 // Whether a batch through one matrix takes the tiled matrix-core kernels (split, product, sum of the K
 // parts: 8-15 us of launches and latency) rather than the GEMV per token, whose time grows with s. The line
 // lies where s * columns * rows repays that, later for a matrix of less than 8 M weights (it stays in an
-// XCD's L2 for the GEMV; less so up to 1024 columns, where a tile's chain is short), earlier for many rows (whole tiles fill the chip) and past 6144 columns, where the
-// GEMV is slower; past 8192 columns the GEMV reads a row per workgroup. us, GEMV against tiled:
+// XCD's L2 for the GEMV; less so up to 1024 columns, where a tile's chain is short), earlier for many rows
+// (whole tiles fill the chip) and past 6144 columns, where the GEMV is slower; past 8192 columns the GEMV
+// reads a row per workgroup. us, GEMV against tiled:
 //   MXFP4 4096 x 4096   s = 6 12.5 / 12.6, 8 13.4 / 12.6, 16 21.6 / 13.1   2048 x 8192  s = 5 11.0 / 10.0
 //         3584 x 3072   s = 8 11.0 / 11.9, 10 13.0 / 11.8                  8192 x 2048  s = 3 16.4 / 12.2
 //         2048 x 2048   s = 24 11.0 / 12.4, 33 14.9 / 12.8                 1024 x 1024  s = 100 12.8 / 12.3
@@ -1019,7 +1021,8 @@ int route_logits_select(rbt_ctx *c, const rbt::RouterArgs &ra, int erows, const 
   const bool al = al16({ra.x, ra.W, sgate}), exact = rbt::router_exact_ok(ra.S, ra.H);
   const bool batch = !exact && rbt::router_batch_ok(ra) && al16({sgate});
   // (where the batch form could run instead, the parts must not be cut to fit the spare rows)
-  const size_t fit = exact ? SIZE_MAX : 4 * spare_n, need = rbt::router_bounded_scratch(ra, erows, batch ? SIZE_MAX : fit);
+  const size_t fit = exact ? SIZE_MAX : 4 * spare_n;
+  const size_t need = rbt::router_bounded_scratch(ra, erows, batch ? SIZE_MAX : fit);
   const bool bounded = ra.S >= rbt::RB_MIN_S && rbt::router_bounded_ok(ra) && al &&
                        (!batch || (long)ra.S * ra.E >= RB_LINE) && need <= fit;
   if (batch && !bounded) {
